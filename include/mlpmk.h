@@ -174,6 +174,23 @@ enum {
 int mlpmk_fwd_launch_info(int num_layers, const int* dims, int dtype, int64_t M, int stash, int* info);
 
 /*
+ * Forward of wider and deeper 16-bit networks than mlpmk_fwd takes: 2..8
+ * layers, input and hidden widths multiples of 8 in [8, 512], output widths in
+ * [1, 512], fp16 or bf16.  Same arguments and results as mlpmk_fwd, plus a
+ * device workspace of at least mlpmk_fwd_layers_workspace_size bytes (16-byte
+ * aligned, contents undefined before and after) for the weights in MFMA
+ * operand order: one launch packs them, a second runs every layer.  The
+ * reference's kernel takes any width (/root/reference/kernel.py:60-123).
+ *
+ * mlpmk_fwd_layers_workspace_size returns MLPMK_ERR_UNSUPPORTED_SHAPE for
+ * networks and element types mlpmk_fwd_layers does not take; it needs no
+ * device.
+ */
+int mlpmk_fwd_layers_workspace_size(int num_layers, const int* dims, int dtype, int64_t* bytes);
+int mlpmk_fwd_layers(int num_layers, const int* dims, int dtype, const void* x, const void* const* w, void* out,
+                     float* const* stash, void* workspace, int64_t workspace_bytes, int64_t M, void* stream);
+
+/*
  * Backward megakernel (one launch): data gradients with MFMA, weight gradients
  * as split-K partials reduced in LDS and then added with global fp32 atomics
  * by every workgroup.  mlpmk_bwd_ws below is the faster form, and the only

@@ -30,6 +30,11 @@ SIGNATURES = {
     "mlpmk_bwd_supported_dtype": (c_int, [c_int, P_INT, c_int]),
     "mlpmk_fwd": (c_int, [c_int, P_INT, c_int, c_void_p, P_VOIDP, c_void_p, P_VOIDP, c_int64, c_void_p]),
     "mlpmk_fwd_launch_info": (c_int, [c_int, P_INT, c_int, c_int64, c_int, P_INT]),
+    "mlpmk_fwd_layers_workspace_size": (c_int, [c_int, P_INT, c_int, ctypes.POINTER(c_int64)]),
+    "mlpmk_fwd_layers": (
+        c_int,
+        [c_int, P_INT, c_int, c_void_p, P_VOIDP, c_void_p, P_VOIDP, c_void_p, c_int64, c_int64, c_void_p],
+    ),
     "mlpmk_bwd": (
         c_int,
         [c_int, P_INT, c_int, c_void_p, P_VOIDP, P_VOIDP, c_void_p, c_int64, c_void_p, P_VOIDP, c_int64, c_void_p],

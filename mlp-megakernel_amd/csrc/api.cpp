@@ -15,6 +15,9 @@ namespace mlpmk {
 bool fwd_supported_dims(int L, const int* dims);
 bool fwd_supported_dtype(int L, const int* dims, int dtype);
 int fwd_dispatch(int L, const int* dims, const FwdParams& p, bool stash, int dtype, hipStream_t st, LaunchInfo* info);
+bool fwd_layers_supported(int L, const int* dims, int dtype);
+int64_t fwd_layers_workspace(int L, const int* dims);
+int fwd_layers_dispatch(int L, const int* dims, const FwdParams& p, bool stash, int dtype, void* ws, hipStream_t st);
 bool bwd_supported_dims(int L, const int* dims);
 bool bwd_supported_dtype(int L, const int* dims, int dtype);
 bool bwd_recompute_supported(int L, const int* dims);
@@ -116,7 +119,7 @@ using namespace mlpmk;
 
 extern "C" {
 
-int mlpmk_version(void) { return 204; }  // 2.04: mlpmk_softplus_f32, mlpmk_fwd_supported_dtype (2.03: MLPMK_BWD_WRITE_DW)
+int mlpmk_version(void) { return 205; }  // 2.05: mlpmk_fwd_layers (2.04: mlpmk_softplus_f32, mlpmk_fwd_supported_dtype 2.03: MLPMK_BWD_WRITE_DW)
 
 const char* mlpmk_status_string(int status) {
   switch (status) {
@@ -159,6 +162,36 @@ int mlpmk_bwd_recompute_supported(int num_layers, const int* dims) {
   return bwd_recompute_supported(num_layers, dims) ? 1 : 0;
 }
 
+// The tensors of a forward call: pointer checks, then FwdParams.  With M == 0
+// only the weights are looked at.
+static int fwd_params(int num_layers, const int* dims, const void* x, const void* const* w, void* out,
+                      float* const* stash, int64_t M, FwdParams* p) {
+  int rc;
+  for (int l = 0; l < num_layers; ++l) {
+    char name[16];
+    snprintf(name, sizeof(name), "w[%d]", l);
+    if ((rc = check_ptr(w[l], name))) return rc;
+    p->w[l] = static_cast<const _Float16*>(w[l]);
+  }
+  if (M == 0) return MLPMK_OK;
+  if ((rc = check_ptr(x, "x"))) return rc;
+  if ((rc = check_ptr(out, "out"))) return rc;
+  if (stash) {
+    for (int l = 0; l < num_layers - 1; ++l) {
+      if (!stash[l]) continue;  // not written
+      char name[16];
+      snprintf(name, sizeof(name), "stash[%d]", l);
+      if ((rc = check_ptr(stash[l], name))) return rc;
+      p->stash[l] = stash[l];
+    }
+  }
+  p->x = static_cast<const _Float16*>(x);
+  p->out = static_cast<_Float16*>(out);
+  p->M = M;
+  for (int l = 0; l <= num_layers; ++l) p->dims[l] = dims[l];
+  return MLPMK_OK;
+}
+
 int mlpmk_fwd(int num_layers, const int* dims, int dtype, const void* x, const void* const* w, void* out,
               float* const* stash, int64_t M, void* stream) {
   g_last_error[0] = 0;
@@ -170,29 +203,39 @@ int mlpmk_fwd(int num_layers, const int* dims, int dtype, const void* x, const v
   if (!fwd_supported_dims(num_layers, dims))
     return fail(MLPMK_ERR_UNSUPPORTED_SHAPE, "no forward kernel for these widths");
   FwdParams p = {};
-  for (int l = 0; l < num_layers; ++l) {
-    char name[16];
-    snprintf(name, sizeof(name), "w[%d]", l);
-    if ((rc = check_ptr(w[l], name))) return rc;
-    p.w[l] = static_cast<const _Float16*>(w[l]);
-  }
+  if ((rc = fwd_params(num_layers, dims, x, w, out, stash, M, &p))) return rc;
   if (M == 0) return MLPMK_OK;
-  if ((rc = check_ptr(x, "x"))) return rc;
-  if ((rc = check_ptr(out, "out"))) return rc;
-  if (stash) {
-    for (int l = 0; l < num_layers - 1; ++l) {
-      if (!stash[l]) continue;  // not written
-      char name[16];
-      snprintf(name, sizeof(name), "stash[%d]", l);
-      if ((rc = check_ptr(stash[l], name))) return rc;
-      p.stash[l] = stash[l];
-    }
-  }
-  p.x = static_cast<const _Float16*>(x);
-  p.out = static_cast<_Float16*>(out);
-  p.M = M;
-  for (int l = 0; l <= num_layers; ++l) p.dims[l] = dims[l];
   return fwd_dispatch(num_layers, dims, p, stash != nullptr, dtype, static_cast<hipStream_t>(stream), nullptr);
+}
+
+int mlpmk_fwd_layers_workspace_size(int num_layers, const int* dims, int dtype, int64_t* bytes) {
+  g_last_error[0] = 0;
+  int rc = check_dims(num_layers, dims);
+  if (rc) return rc;
+  if ((rc = check_fwd_dtype(dtype))) return rc;
+  if (!bytes) return fail(MLPMK_ERR_INVALID_ARG, "bytes is NULL");
+  if (!fwd_layers_supported(num_layers, dims, dtype))
+    return fail(MLPMK_ERR_UNSUPPORTED_SHAPE, "no forward kernel for these widths and dtype");
+  *bytes = fwd_layers_workspace(num_layers, dims);
+  return MLPMK_OK;
+}
+
+int mlpmk_fwd_layers(int num_layers, const int* dims, int dtype, const void* x, const void* const* w, void* out,
+                     float* const* stash, void* workspace, int64_t workspace_bytes, int64_t M, void* stream) {
+  int64_t need = 0;
+  int rc = mlpmk_fwd_layers_workspace_size(num_layers, dims, dtype, &need);
+  if (rc) return rc;
+  if (M < 0) return fail(MLPMK_ERR_INVALID_ARG, "M=%lld is negative", (long long)M);
+  if (!w) return fail(MLPMK_ERR_INVALID_ARG, "w is NULL");
+  FwdParams p = {};
+  if ((rc = fwd_params(num_layers, dims, x, w, out, stash, M, &p))) return rc;
+  if (M == 0) return MLPMK_OK;
+  if ((rc = check_ptr(workspace, "workspace"))) return rc;
+  if (workspace_bytes < need)
+    return fail(MLPMK_ERR_INVALID_ARG, "workspace_bytes=%lld; %lld needed", (long long)workspace_bytes,
+                (long long)need);
+  return fwd_layers_dispatch(num_layers, dims, p, stash != nullptr, dtype, workspace,
+                             static_cast<hipStream_t>(stream));
 }
 
 int mlpmk_fwd_launch_info(int num_layers, const int* dims, int dtype, int64_t M, int stash, int* info) {

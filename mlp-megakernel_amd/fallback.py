@@ -32,10 +32,13 @@ fp32 for fp32 tensors).
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
+import torch.nn.functional as F
 
 from . import _lib
-from .ops import _check, _elem_code, _launch
+from .ops import _check, _elem_code, _fwd_code, _launch
 
 
 def sigmoid_h_mul(h, dh, dz16_dtype=None):
@@ -71,14 +74,68 @@ def softplus_f32(z, out=None):
     return h
 
 
+_layers_ws = {}  # (widths, dtype) -> workspace bytes of mlpmk_fwd_layers, -1 where it takes no such network
+
+
+def _layers_workspace(dims, dtype):
+    key = (dims, dtype)
+    n = _layers_ws.get(key)
+    if n is None:
+        out = ctypes.c_int64(-1)
+        if dtype != torch.float32:
+            rc = _lib.get().mlpmk_fwd_layers_workspace_size(len(dims) - 1, _lib.dims_array(dims), _fwd_code(dtype),
+                                                            ctypes.byref(out))
+            if rc not in (0, 2):  # MLPMK_ERR_UNSUPPORTED_SHAPE: -1 stays
+                _check("mlpmk_fwd_layers_workspace_size", rc)
+        n = _layers_ws[key] = out.value
+    return n
+
+
+def _fwd_layers(x, weights, stash):
+    """:func:`fwd` through ``mlpmk_fwd_layers``, or None where that kernel does
+    not take the call (fp32 tensors, widths above 512, more than 8 layers,
+    hidden widths that are not multiples of 8, tensors off a 16-byte
+    boundary).  An input width that is not a multiple of 8 is padded with zero
+    columns of x and zero rows of W_1, which add nothing to the product."""
+    if x.dim() != 2 or any(w.dim() != 2 for w in weights):
+        return None
+    dims = (int(x.shape[1]),) + tuple(int(w.shape[1]) for w in weights)
+    pad = -dims[0] % 8
+    dims = (dims[0] + pad,) + dims[1:]
+    if x.device.type != "cuda" or any(w.device != x.device for w in weights):
+        return None
+    nbytes = _layers_workspace(dims, x.dtype)
+    if nbytes < 0 or any(tuple(w.shape) != (k, n) for w, k, n in zip(weights, (dims[0] - pad,) + dims[1:], dims[1:])):
+        return None
+    x, weights = x.contiguous(), [w.contiguous() for w in weights]
+    if pad:
+        x, weights[0] = F.pad(x, (0, pad)), F.pad(weights[0], (0, 0, 0, pad))
+    if x.data_ptr() % 16 or any(w.data_ptr() % 16 for w in weights):
+        return None
+    dev, M = x.device, int(x.shape[0])
+    out = torch.empty((M, dims[-1]), dtype=x.dtype, device=dev)
+    hs = [torch.empty((M, d), dtype=torch.float32, device=dev) for d in dims[1:-1]] if stash else None
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    L = len(weights)
+    rc = _launch(dev, _lib.get().mlpmk_fwd_layers, L, _lib.dims_array(dims), _fwd_code(x.dtype), x.data_ptr(),
+                 (_lib.c_void_p * L)(*[w.data_ptr() for w in weights]), out.data_ptr(),
+                 (_lib.c_void_p * (L - 1))(*[h.data_ptr() for h in hs]) if stash else None, ws.data_ptr(), nbytes, M)
+    _check("mlpmk_fwd_layers", rc)
+    return (out, hs) if stash else out
+
+
 def fwd(x, weights, stash=False):
-    """Forward layer by layer, for the networks no fused forward takes: fp32
-    tensors wider than 128, any tensors wider than 256, more than 5 layers,
-    hidden widths that are not multiples of 16.  ``z = a @ W_l``
+    """Forward for the networks no megakernel takes: fp32 tensors wider than
+    128, any tensors wider than 256, more than 5 layers, hidden widths that
+    are not multiples of 16.  16-bit networks up to 512 wide and 8 layers deep
+    run in one launch (``mlpmk_fwd_layers``, after one that packs the weights;
+    128-512-512-128 in fp16 at 16,384 rows 182 us layer by layer, 25 us).
+    The others run layer by layer: ``z = a @ W_l``
     as an fp32 library GEMM (rocBLAS / hipBLASLt through torch; 16-bit
     values are exact in fp32, so this is the fused kernels' fp32
-    accumulation), then the fp32 softplus kernel on every hidden layer, whose
-    output is rounded to the tensor format before the next GEMM as the
+    accumulation), then the fp32 softplus kernel on every hidden layer.
+    Either way the hidden h is
+    rounded to the tensor format before the next layer as the
     reference's kernel rounds its h (kernel.py:110,117).  The reference's
     kernels take any width (kernel.py:60-63; INPUT_DTYPE = fp32,
     mlp_fused.md:159-166).  Returns ``out`` in x's dtype, or ``(out, [h1 ..
@@ -86,6 +143,9 @@ def fwd(x, weights, stash=False):
     dt = x.dtype
     if dt not in (torch.float32, torch.float16, torch.bfloat16) or any(w.dtype != dt for w in weights):
         raise ValueError("x and the weights must share one of fp32, fp16 or bf16")
+    res = _fwd_layers(x, weights, stash)
+    if res is not None:
+        return res
     a = x.contiguous() if dt == torch.float32 else x.float()
     hs = []
     with torch.autocast("cuda", enabled=False):  # the GEMMs stay fp32 under a caller's autocast

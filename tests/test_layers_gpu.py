@@ -1,0 +1,145 @@
+"""``mlpmk_fwd_layers``: the one-launch forward of 16-bit networks wider than
+256 or deeper than 5 layers (csrc/fwd_layers.hip), through ``fallback.fwd``,
+against the CPU oracle (/root/reference/kernel.py:60-123 takes any width).
+
+Sizes where the kernel changes its split: tiles of 32 and 64 rows and their
+remainders, feature groups of 64 (widths just above a multiple, layers of at
+most half or a quarter of the workgroup's features), ragged output widths and
+inputs that are padded to a multiple of 8.  Tolerances are those of the other
+16-bit forwards: fp16 outputs and activations within 1e-2 + 1e-2 |ref| of the
+oracle that rounds h to fp16 between layers, bf16 within 3e-2.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from mlpmk import _lib, fallback, ops
+from oracle import mlp_oracle as orc
+
+A = 1 << 20  # a 16-byte aligned address that is never read
+
+
+def _workspace(dims, code):
+    n = ctypes.c_int64(-1)
+    p, _k = _lib.int_array(list(dims))
+    return _lib.get().mlpmk_fwd_layers_workspace_size(len(dims) - 1, p, code, ctypes.byref(n)), n.value
+
+
+@pytest.mark.parametrize("dims,code,want", [
+    ((128, 512, 512, 128), 1, 2 * (128 * 512 + 512 * 512 + 512 * 128)),
+    ((8, 8, 1), 2, 2 * 2 * 64 * 64),
+    ((72, 100, 5), 1, None),            # a hidden width that is no multiple of 8
+    ((128, 520, 128), 1, None),
+    ((128, 512, 513), 2, None),
+    ((128, 512, 128), 0, None),         # fp32 tensors
+    ((16,) * 10, 1, None),              # nine layers
+])
+def test_workspace_and_supported_shapes(dims, code, want):
+    rc, n = _workspace(dims, code)
+    assert (rc, n) == ((0, want) if want is not None else (2, -1))
+
+
+def test_validation_before_any_launch():
+    lib = _lib.get()
+    dims = (128, 512, 128)
+    pd, _k = _lib.int_array(list(dims))
+    w = (_lib.c_void_p * 2)(A, A)
+    need = _workspace(dims, 1)[1]
+
+    def call(x=A, out=A, ws=A, nb=need, m=4, wp=w):
+        return lib.mlpmk_fwd_layers(2, pd, 1, x, wp, out, None, ws, nb, m, None)
+
+    assert call(m=0) == 0
+    assert call(m=-1) == 1 and call(x=None) == 1 and call(out=A + 2) == 3 and call(wp=None) == 1
+    assert call(ws=None) == 1 and call(nb=need - 1) == 1 and call(ws=A + 8) == 3
+
+
+SHAPES = [
+    ((128, 512, 512, 128), [1, 31, 64, 65, 8192, 8193, 20000]),
+    ((128, 272, 272, 128), [33, 1000]),
+    ((64, 320, 24, 8), [129]),              # a quarter of the features, then one feature group
+    ((200, 512, 448), [97]),                # output width above a whole number of groups
+    ((16, 264, 264, 264, 3), [257]),        # ragged output, widths just above 256
+    ((128, 512, 511), [70]),
+    ((3, 512, 512, 4), [100, 9000]),        # padded input
+    ((32,) * 9, [300]),                     # eight layers
+    ((8, 8, 1), [5]),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims,m", [(d, m) for d, ms in SHAPES for m in ms])
+@pytest.mark.parametrize("elem", ["f16", "bf16"])
+def test_layers_forward_and_stash_match_oracle(dims, m, elem):
+    tol, dt = (1e-2, torch.float16) if elem == "f16" else (3e-2, torch.bfloat16)
+    kw = {} if elem == "f16" else {"elem": "bf16"}
+    x, ws = orc.make_inputs(dims, m, seed=m + len(dims), **kw)
+    xd = torch.from_numpy(x).cuda().to(dt)
+    wd = [torch.from_numpy(w).cuda().to(dt) for w in ws]
+    res = fallback._fwd_layers(xd, wd, True)
+    assert res is not None, "the kernel takes this network"
+    out, hs = res
+    ref, ref_h = orc.forward(x, ws, round_hidden=True, return_hidden=True, **kw)
+    ok, err, _ = orc.allclose_report(out.float().cpu().numpy(), ref, tol, tol)
+    assert ok, f"out: max|err| {err}"
+    for i, (h, r) in enumerate(zip(hs, ref_h)):
+        ok, err, _ = orc.allclose_report(h.cpu().numpy(), r, tol, tol)
+        assert ok, f"h{i + 1}: max|err| {err}"
+    assert torch.equal(fallback.fwd(xd, wd), out)  # inference: the same bits
+    # the tile size changes no bit
+    head = min(m, 40)
+    assert torch.equal(fallback.fwd(xd[:head], wd), out[:head])
+
+
+@pytest.mark.gpu
+def test_layers_large_and_nonfinite_rows():
+    dims, m = (128, 320, 320, 128), 500
+    x, ws = orc.make_inputs(dims, m, seed=3)
+    big = np.arange(m) % 7 == 0
+    x[big] = (x[big].astype(np.float32) * 300.0).astype(np.float16)
+    x[5, 3], x[300, 0] = np.inf, np.nan
+    out = fallback.fwd(torch.from_numpy(x).cuda(), [torch.from_numpy(w).cuda() for w in ws]).float().cpu().numpy()
+    ref = orc.forward(x, ws, round_hidden=True)
+    bad = np.zeros(m, bool)
+    bad[[5, 300]] = True
+    assert not np.isfinite(out[bad]).any() and np.isfinite(out[~bad]).all()
+    ok, err, _ = orc.allclose_report(out[~bad & ~big], ref[~bad & ~big], 1e-2, 1e-2)
+    assert ok, err
+    assert np.abs(out[big] - ref[big]).max() <= 2e-3 * np.abs(ref[big]).max()
+
+
+@pytest.mark.gpu
+def test_layers_small_activations_keep_their_digits():
+    # softplus(z) = e^z (1 - e^z / 2 ...) for z << 0: the fp32 stash within a
+    # few ulp of the float64 value of the same fp32 z (z = x w exactly: one
+    # input feature), as the elementwise kernel of the layer-by-layer path is.
+    # |z| log2 e rounded to fp32 moves e^z by |z| 2^-24 relative: 1.2e-6 at 20.
+    z = torch.linspace(-20, 24, 352, device="cuda").bfloat16()
+    x = torch.zeros((4, 8), device="cuda", dtype=torch.bfloat16)
+    x[:, 0] = 1
+    w0 = torch.zeros((8, 352), device="cuda", dtype=torch.bfloat16)
+    w0[0] = z
+    _, (h,) = fallback.fwd(x, [w0, torch.zeros((352, 8), device="cuda", dtype=torch.bfloat16)], stash=True)
+    ref = torch.log1p(torch.exp(z.double()))
+    assert ((h[0].double() - ref).abs() / ref).max().item() < 2e-6
+
+
+@pytest.mark.gpu
+def test_calls_the_kernel_does_not_take_still_run():
+    # off a 16-byte boundary, fp32, a hidden width that is no multiple of 8, a
+    # batch of more than two dimensions: the library-GEMM route, as before
+    g = torch.Generator(device="cuda").manual_seed(0)
+    flat = torch.randn(1 + 50 * 128, generator=g, device="cuda").half()
+    x = flat[1:].view(50, 128)
+    ws = [(torch.randn(s, generator=g, device="cuda") / 16).half() for s in ((128, 512), (512, 64))]
+    assert fallback._fwd_layers(x, ws, False) is None
+    assert fallback._fwd_layers(x.float(), [w.float() for w in ws], False) is None
+    assert fallback._fwd_layers(x, [ws[0][:, :300].contiguous(), ws[1][:300]], False) is None
+    x3 = x.reshape(2, 25, 128)
+    assert fallback._fwd_layers(x3, ws, False) is None
+    ref = torch.nn.functional.softplus(x.double() @ ws[0].double()) @ ws[1].double()
+    for got in (fallback.fwd(x, ws), fallback.fwd(x.clone(), ws), fallback.fwd(x3, ws).reshape(50, 64)):
+        torch.testing.assert_close(got.double(), ref, atol=1e-2, rtol=1e-2)
+    assert ops.fwd_supported([128, 512, 64]) is False
