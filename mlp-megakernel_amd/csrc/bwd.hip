@@ -1305,15 +1305,19 @@ static int bwd_split_workspace(int L, const int* dims, int64_t M, bool dx, int64
   return MLPMK_OK;
 }
 
+// mlpmk_bwd takes up to 3 layers, whatever the kernel behind it.
+static int no_split_workspace() {
+  return fail(MLPMK_ERR_INVALID_ARG,
+              "a backward of more than 3 layers passes dz between two launches through the workspace: "
+              "use mlpmk_bwd_ws");
+}
+
 template <class TOP, class BOT>
 static int launch_bwd_split(const BwdParams& p, int L, hipStream_t st) {
   constexpr int S = BOT::L;
   static_assert(TOP::L >= 2 && S >= 2, "segment shapes");
   if (L != TOP::L + S) return fail(MLPMK_ERR_UNSUPPORTED_SHAPE, "split backward: %d layers", L);
-  if (!p.part)
-    return fail(MLPMK_ERR_INVALID_ARG,
-                "a backward of more than 3 layers passes dz between two launches through the workspace: "
-                "use mlpmk_bwd_ws");
+  if (!p.part) return no_split_workspace();
   char* const ws = reinterpret_cast<char*>(p.part);
   _Float16* const dzs = reinterpret_cast<_Float16*>(ws);
   float* const part = reinterpret_cast<float*>(ws + dz_bytes(p.M));
@@ -1357,6 +1361,34 @@ static int launch_bwd_split(const BwdParams& p, int L, hipStream_t st) {
 typedef Gen<BNet2L128> GBNet2;
 typedef Gen<BNet3L128> GBNet3;
 
+// The same compiled at width 64, for networks whose layers all fit it: a
+// quarter of the MFMAs and of the accumulators, so that every depth runs in
+// one launch.
+template <int L>
+struct GB64;
+template <>
+struct GB64<2> {
+  typedef Gen<Net<64, 64, 64>> type;
+};
+template <>
+struct GB64<3> {
+  typedef Gen<Net<64, 64, 64, 64>> type;
+};
+template <>
+struct GB64<4> {
+  typedef Gen<Net<64, 64, 64, 64, 64>> type;
+};
+template <>
+struct GB64<5> {
+  typedef Gen<Net<64, 64, 64, 64, 64, 64>> type;
+};
+
+static bool bwd_w64_dims(int L, const int* dims) {
+  for (int i = 0; i <= L; ++i)
+    if (dims[i] > 64) return false;
+  return true;
+}
+
 bool bwd_generic_dims(int L, const int* dims) {
   if (L < 2 || L > 5) return false;
   for (int i = 0; i < L; ++i)
@@ -1399,6 +1431,14 @@ static int bwd_workspace_t(int L, const int* dims, int64_t M, bool dx, int64_t* 
   }
   if (bdims_match<BNetNarrow>(L, dims)) return bwd_workspace_any<NN>(M, dx, we, bytes);
   if (bwd_generic_dims(L, dims)) {
+    if (bwd_w64_dims(L, dims)) {
+      switch (L) {
+        case 2: return bwd_workspace_any<typename ElemNet<B, GB64<2>::type>::type>(M, dx, we, bytes);
+        case 3: return bwd_workspace_any<typename ElemNet<B, GB64<3>::type>::type>(M, dx, we, bytes);
+        case 4: return bwd_workspace_any<typename ElemNet<B, GB64<4>::type>::type>(M, dx, we, bytes);
+        default: return bwd_workspace_any<typename ElemNet<B, GB64<5>::type>::type>(M, dx, we, bytes);
+      }
+    }
     switch (L) {
       case 2: return bwd_workspace_any<G2>(M, dx, we, bytes);
       case 3: return bwd_workspace_any<G3>(M, dx, we, bytes);
@@ -1523,6 +1563,15 @@ static int bwd_dispatch_t(int L, const int* dims, const BwdParams& p, hipStream_
   if (bdims_match<BNet5L128>(L, dims)) return launch_bwd_split<N2, N3>(p, L, st);
   if (bdims_match<BNetNarrow>(L, dims)) return launch_bwd_any<NN>(p, st);
   if (bwd_generic_dims(L, dims)) {
+    if (bwd_w64_dims(L, dims)) {
+      if (L > 3 && !p.part) return no_split_workspace();
+      switch (L) {
+        case 2: return launch_bwd_any<typename ElemNet<B, GB64<2>::type>::type>(p, st);
+        case 3: return launch_bwd_any<typename ElemNet<B, GB64<3>::type>::type>(p, st);
+        case 4: return launch_bwd_any<typename ElemNet<B, GB64<4>::type>::type>(p, st);
+        default: return launch_bwd_any<typename ElemNet<B, GB64<5>::type>::type>(p, st);
+      }
+    }
     switch (L) {
       case 2: return launch_bwd_any<G2>(p, st);
       case 3: return launch_bwd_any<G3>(p, st);

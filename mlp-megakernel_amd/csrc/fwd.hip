@@ -42,6 +42,8 @@ bool fwd_supported_dtype(int L, const int* dims, int dtype) {
 int fwd_split_dispatch(int L, const int* dims, const FwdParams& p, bool stash, bool bf, hipStream_t st, int cus,
                        LaunchInfo* info);
 
+int fwd_w64_dispatch(int L, const FwdParams& p, bool stash, bool bf, hipStream_t st, LaunchInfo* info);
+
 // B: bf16 tensors (every shape is instantiated for both element formats).
 template <bool B>
 static int fwd_dispatch_t(int L, const int* dims, const FwdParams& p, bool stash, hipStream_t st, LaunchInfo* info) {
@@ -52,6 +54,10 @@ static int fwd_dispatch_t(int L, const int* dims, const FwdParams& p, bool stash
   if (dims_match<NetNarrow>(L, dims))
     return launch_fwd_any<typename ElemNet<B, NetNarrow>::type, 2, 16, 1, 16, 1>(p, stash, st, info);
   if (fwd_generic_dims(L, dims)) {
+    // Kernels compiled at width 64 where no layer is wider (fwd_w64.hip).
+    int wmax = 0;
+    for (int i = 0; i <= L; ++i) wmax = dims[i] > wmax ? dims[i] : wmax;
+    if (wmax <= 64) return fwd_w64_dispatch(L, p, stash, B, st, info);
     switch (L) {
       // At most 8 waves (4 for the 5-layer stash kernel): the runtime
       // strides cannot fold into immediate offsets, and the 12-wave kernels
