@@ -1039,8 +1039,11 @@ struct BwdWave {
 };
 
 
+// The runtime-width kernels of at most 64 features keep two waves per SIMD:
+// left to itself the allocator spread over the accumulation registers and one
+// wave (16-64-64-64-4 in fp16 at 262,144 rows 79 -> 71 us).
 template <class N, int NW, bool DX, bool SEG>
-__global__ __launch_bounds__(NW * 64) void bwd_kernel(BwdParams p) {
+__global__ __launch_bounds__(NW * 64, N::gen && N::ksmax() <= 4 ? 2 : 1) void bwd_kernel(BwdParams p) {
   using Gm = BwdGeom<N, NW, DX, SEG>;
   static_assert(Gm::valid(), "unsupported backward shape");
   constexpr int R = Gm::R;
@@ -1363,7 +1366,8 @@ typedef Gen<BNet3L128> GBNet3;
 
 // The same compiled at width 64, for networks whose layers all fit it: a
 // quarter of the MFMAs and of the accumulators, so that every depth runs in
-// one launch.
+// one launch (16-64-64-64-4 in fp16 at 262,144 rows, 128-wide in two launches
+// -> 64-wide: 166 -> 71 us; 48-wide 3-layer with dx at 100,000: 66 -> 32).
 template <int L>
 struct GB64;
 template <>
