@@ -83,10 +83,12 @@ struct DgGeo {
     for (int l = LO; l < L; ++l) m = ks(l) > m ? ks(l) : m;
     return m;
   }
-  // Exchange tile width (features per row; a power of two for the swizzle):
-  // layer l >= LO + 1 hands dz_{l-1} (d[l] features) to layer l - 1.
+  // Exchange tile width (features per row; a power of two for the swizzle, of
+  // whole 64-feature K turns): dL/dout (d[L] features), and layer l >= LO + 1
+  // hands dz_{l-1} (d[l] features) to layer l - 1.
   static constexpr int tw() {
-    int m = 32;
+    int m = 64;
+    while (m < N::d[L]) m *= 2;
     for (int l = LO + 1; l < L; ++l)
       while (m < N::d[l]) m *= 2;
     return m;
@@ -99,273 +101,274 @@ struct DgGeo {
   }
 };
 
+// A workgroup of NWV waves runs tiles of 32 RB rows, one after the other; wave w
+// owns features [32w, 32w + 32) of every data gradient and all rows of the
+// tile.  dL/dout and every dz_l go through LDS tiles (two, in turns: one
+// barrier per layer), from which each wave reads its B operands a K-step ahead
+// of the MFMA that takes them.  Everything that comes from memory is requested
+// a tile ahead: the next tile's dL/dout (each thread a share of it) right after
+// this tile's went into LDS, the next tile's h_l into the registers that this
+// tile's sigma(h_l) just left.
+//
 // RES: every layer's fragments stay in registers for the whole kernel
-// (loaded once per workgroup); otherwise (widths above 128, whose fragments
-// would not fit beside the rest) each layer's are read from L2 right before
-// its MFMA chain, every block -- except, in the 16-bit kernels of widths up
-// to 256 (STG), those of the data-gradient layer with the most weights: each
-// wave copies its own into LDS once (NWV x 16 K-steps x 1 KiB = 128 KiB,
-// beside the 32 KiB exchange tiles: the workgroup's whole 160 KiB, which its
-// registers already hold to one workgroup per CU) and reads them from there.
-// 128-256-256-128 at 131072 rows: L2 reads of fragments per 32-row block
-// 192 -> 64 KiB.
-template <class N, int EM, bool DX, bool RES>
+// (loaded once per workgroup); otherwise they are read from L2 through a ring
+// of kRing K-steps, the next layer's first ones requested before this layer's
+// results are evaluated.
+template <class N, int EM, bool DX, bool RES, int RB>
 struct DgWave {
   using G = DgGeo<N, DX>;
   static constexpr int L = N::L, CH = G::CH, NT = EM == EM_F32 ? 2 : 1;
-  static constexpr bool STG = !RES && EM != EM_F32 && G::NWV == 8;
-  static constexpr int STG_ELEMS = STG ? G::NWV * G::KSM * 64 : 1;  // f16x8 payloads
+  static constexpr int ROWS = 32 * RB;
+  static constexpr int kRing = 4;
+  static constexpr uint32_t kPast = 0x80000000u;  // past every resource: loads read zeros
+  // dL/dout pieces (8 elements) of a tile per thread.
+  static constexpr int OCH = (N::d[L] + 63) / 64 * 8;  // pieces of a row, padded to whole K turns
+  static constexpr int PD = (ROWS * OCH + G::NWV * 64 - 1) / (G::NWV * 64);
+  struct Raw {  // 8 tensor elements as loaded
+    f32x4 v[NT];
+  };
   const TpParams& p;
-  f16x8 (*tile)[NT][32 * CH];  // [2][NT][32 * CH]
+  f16x8 (*tile)[NT][ROWS * CH];  // [2][NT][ROWS * CH]
   int lane, n, g, w;
-  f16x8* stg = nullptr;               // STG: [NWV][KSM][64] fragments of layer stg_l
-  int stg_l = -1;
-  int par = 0;                        // exchange tile of the next hand-over
-  Opnd fr[RES ? L : 1][G::KSM];       // this wave's A fragments (output block w)
-  Opnd B[G::KSM];                     // B operands of the current layer: dz_l of row n
-  float h[L][16];                     // h_l of this wave's 16 features of row n (l >= 1)
-  float hn[RES ? L : 1][16];          // RES: the same for the workgroup's next block, in flight
+  int par = 0;                          // tile of the next hand-over
+  Opnd fr[RES ? L : 1][RES ? G::KSM : 1];  // RES: this wave's A fragments (output block w)
+  Raw ring[RES ? 1 : kRing];            // !RES: the next K-steps' fragments
+  Raw dr[PD];                           // the next tile's dL/dout
+  float h[L][RB][16];                   // h_l of this wave's 16 features of row n of each block (l >= 1)
 
   __device__ __forceinline__ bool owns(int l) const { return 32 * w < dimw<N>(p, l); }
+  __device__ __forceinline__ static Raw load_raw(rsrc_t r, uint32_t byte) {
+    Raw v;
+#pragma unroll
+    for (int i = 0; i < NT; ++i) v.v[i] = buf_load16<f32x4>(r, byte + 16 * i);
+    return v;
+  }
+  __device__ __forceinline__ static Opnd to_op(const Raw& v) {
+    if constexpr (EM == EM_F32) {
+      const f32x4 a = v.v[0], b = v.v[NT - 1];
+      const float f[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+      return make_op<EM>(f);
+    } else {
+      return Opnd{__builtin_bit_cast(f16x8, v.v[0]), f16x8{}};
+    }
+  }
 
   // Fragment (block w, K-step s) of layer l: lane (i, g) holds
-  // W_l[outfeat(w, i)][16s + 8g + 0..7].  Rows past the true width read
-  // zeros through the resource; columns past it are masked (Gen).
+  // W_l[outfeat(w, i)][16s + 8g + 0..7].  Rows and columns past the true
+  // widths read zeros (offsets past the resource).
   template <int l>
-  __device__ __forceinline__ void load_frags(Opnd (&f)[G::KSM]) const {
+  __device__ __forceinline__ Raw load_frag(int s) const {
     const int K = dimw<N>(p, l), Nout = dimw<N>(p, l + 1);
     const rsrc_t r = make_rsrc(p.w[l], (uint32_t)(K * Nout * kEs<EM>));
-    const int row = outfeat(w, n);
-#pragma unroll
-    for (int s = 0; s < G::ks(l); ++s) {
-      const int c = 16 * s + 8 * g;
-      if (N::gen && 16 * s >= Nout) {  // a whole K-step past the true width: no load
-        f[s] = Opnd{f16x8{}, f16x8{}};
-        continue;
-      }
-      f[s] = load_op<EM>(r, (uint32_t)(row * Nout + c));
-      if (N::gen && c >= Nout) f[s] = Opnd{f16x8{}, f16x8{}};
-    }
+    const int c = 16 * s + 8 * g;
+    const uint32_t off = (uint32_t)(outfeat(w, n) * Nout + c) * kEs<EM>;
+    return load_raw(r, !N::gen || c < Nout ? off : kPast);
   }
-  // STG: copies this wave's fragments of the data-gradient layer with the
-  // most weights (true widths) into its LDS slots.
-  __device__ __forceinline__ void stage_largest() {
-    int64_t best = 0;
-    for (int l = G::LO; l < L; ++l) {
-      const int64_t e = (int64_t)dimw<N>(p, l) * dimw<N>(p, l + 1);
-      if (e > best) {
-        best = e;
-        stg_l = l;
-      }
-    }
-    stage_layer<G::LO>();
-  }
-  template <int l>
-  __device__ __forceinline__ void stage_layer() {
-    if constexpr (l < L) {
-      if (l == stg_l && owns(l)) {
-        Opnd f[G::KSM];
-        load_frags<l>(f);
-#pragma unroll
-        for (int s = 0; s < G::ks(l); ++s) stg[(w * G::KSM + s) * 64 + lane] = f[s].h;
-      }
-      stage_layer<l + 1>();
-    }
-  }
-  // Layer l's fragments: from the LDS copy if it holds them, else from L2.
-  template <int l>
-  __device__ __forceinline__ void frags_of(Opnd (&f)[G::KSM]) const {
-    if (STG && l == stg_l) {
-      const int Nout = dimw<N>(p, l + 1);
-#pragma unroll
-      for (int s = 0; s < G::ks(l); ++s) {
-        f[s].h = (N::gen && 16 * s >= Nout) ? f16x8{} : stg[(w * G::KSM + s) * 64 + lane];
-        f[s].l = f16x8{};
-      }
-      return;
-    }
-    load_frags<l>(f);
-  }
-
   template <int l = G::LO>
   __device__ __forceinline__ void load_all_frags() {
     if constexpr (l < L) {
-      if (owns(l)) load_frags<l>(fr[l]);
+      if (owns(l)) {
+#pragma unroll
+        for (int s = 0; s < G::ks(l); ++s) fr[l][s] = to_op(load_frag<l>(s));
+      }
       load_all_frags<l + 1>();
     }
   }
+  template <int l>
+  __device__ __forceinline__ void request() {
+    if constexpr (!RES) {
+#pragma unroll
+      for (int t = 0; t < kRing; ++t) {
+        ring[t] = load_frag<l>(t);
+        __builtin_amdgcn_sched_barrier(0);  // in this order: the K loop counts them
+      }
+    }
+  }
 
-  // dL/dout rows from row0 as B operands (K-steps over the output width).
-  // Row stride 0 broadcasts row 0; a negative one (MLPMK_DOUT_SCALAR) one
-  // element to every row and feature below the output width.
+  // dL/dout of the tile at row0: piece q = tid + k * threads is row q / OCH,
+  // elements 8 (q % OCH) .. + 7.  Row stride 0 broadcasts row 0; a negative one
+  // (MLPMK_DOUT_SCALAR) one element to every row and feature below the output
+  // width.  Rows past the batch and features past the width read zeros.
   __device__ __forceinline__ void load_dout(int64_t row0) {
-    constexpr int KS = G::ks(L - 1);
     const int OW = dimw<N>(p, L);
     const int64_t st = p.dout_stride;
-    const uint32_t nr = rows_at(p.M, row0, 32);
-    if (st < 0) {
-      float v;
-      const rsrc_t r1 = make_rsrc(p.dout, nr ? (uint32_t)kEs<EM> : 0u);
-      if constexpr (EM == EM_F32)
-        v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r1, 0, 0, 0));
-      else
-        v = elem_to_f32<kBf<EM>>(__builtin_bit_cast(f16, __builtin_amdgcn_raw_buffer_load_b16(r1, 0, 0, 0)));
-      const float vv[8] = {v, v, v, v, v, v, v, v};
-      const Opnd o = make_op<EM>(vv);
+    const uint32_t nr = rows_at(p.M, row0, ROWS);
+    const bool scalar = st < 0;
+    const int64_t str = st > 0 ? st : 0;
+    const uint32_t bytes = !nr ? 0u : scalar ? (uint32_t)kEs<EM> : (uint32_t)(((nr - 1) * str + OW) * kEs<EM>);
+    const rsrc_t r = make_rsrc(static_cast<const char*>(p.dout) + row0 * str * kEs<EM>, bytes);
 #pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        B[s] = o;
-        if (N::gen && 16 * s + 8 * g >= OW) B[s] = Opnd{f16x8{}, f16x8{}};
+    for (int k = 0; k < PD; ++k) {
+      const int q = (int)threadIdx.x + k * G::NWV * 64, row = q / OCH, c = 8 * (q % OCH);
+      const bool ok = (uint32_t)row < nr && c < OW;
+      if (scalar) {
+        if constexpr (EM == EM_F32) {
+          const float v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, ok ? 0 : (int)kPast, 0, 0));
+          dr[k].v[0] = dr[k].v[NT - 1] = f32x4{v, v, v, v};
+        } else {
+          const int v = (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(r, ok ? 0 : (int)kPast, 0, 0);
+          const int vv = v | (v << 16);
+          dr[k].v[0] = __builtin_bit_cast(f32x4, (i32x4){vv, vv, vv, vv});
+        }
+      } else {
+        dr[k] = load_raw(r, ok ? (uint32_t)(row * str + c) * kEs<EM> : kPast);
       }
-      return;
     }
-    const uint32_t bytes = nr ? (uint32_t)(((int64_t)(nr - 1) * st + OW) * kEs<EM>) : 0u;
-    const rsrc_t r = make_rsrc(static_cast<const char*>(p.dout) + row0 * st * kEs<EM>, bytes);
+  }
+  __device__ __forceinline__ void commit_dout() {
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const int c = 16 * s + 8 * g;
-      B[s] = load_op<EM>(r, (uint32_t)(n * st + c));
-      if (N::gen && c >= OW) B[s] = Opnd{f16x8{}, f16x8{}};
+    for (int k = 0; k < PD; ++k) {
+      const int q = (int)threadIdx.x + k * G::NWV * 64, row = q / OCH, c = q % OCH;
+      if (ROWS * OCH % (G::NWV * 64) != 0 && row >= ROWS) continue;
+      const Opnd o = to_op(dr[k]);
+      tile[par][0][slot<CH>(row, c)] = o.h;
+      if constexpr (NT == 2) tile[par][NT - 1][slot<CH>(row, c)] = o.l;
     }
   }
 
-  // h_l for this wave's 16 features of row n (features 32w + 8g + [0..7]
-  // and 32w + 16 + 8g + [0..7]), fp32.  With RES every stash layer's are
-  // issued at once, a block ahead (into hn, which becomes h when that block
-  // starts: the loads of block b + grid are in flight while block b
-  // computes); otherwise each layer's with its fragments.  Past the batch the
+  // h_l for this wave's 16 features of row n of each row block (features 32w +
+  // 8g + [0..7] and 32w + 16 + 8g + [0..7]), fp32.  Past the batch the
   // resource is empty and the loads return zeros.
-  template <int l = 1>
-  __device__ __forceinline__ void load_h(int64_t row0, float (&dst)[L][16]) {
-    if constexpr (l < L) {
-      load_h_one<l>(row0, dst);
-      load_h<l + 1>(row0, dst);
-    }
-  }
-  __device__ __forceinline__ void take_next_h() {
-    if constexpr (RES) {
-#pragma unroll
-      for (int l = 1; l < L; ++l)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) h[l][j] = hn[l][j];
-    }
-  }
   template <int l>
-  __device__ __forceinline__ void load_h_one(int64_t row0, float (&dst)[L][16]) {
-    {
-      const int HW = dimw<N>(p, l);
-      const rsrc_t r = make_rsrc(p.stash[l - 1] + row0 * HW, owns(l) ? rows_at(p.M, row0, 32) * HW * 4u : 0u);
-      const uint32_t e = (uint32_t)(n * HW + 32 * w + 8 * g) * 4;
-      const f32x4 a = buf_load16<f32x4>(r, e), b = buf_load16<f32x4>(r, e + 16);
-      const f32x4 c = buf_load16<f32x4>(r, e + 64), d = buf_load16<f32x4>(r, e + 80);
+  __device__ __forceinline__ void load_h(int64_t row0) {
+    const int HW = dimw<N>(p, l);
+    const rsrc_t r = make_rsrc(p.stash[l - 1] + row0 * HW, owns(l) ? rows_at(p.M, row0, ROWS) * HW * 4u : 0u);
+#pragma unroll
+    for (int b = 0; b < RB; ++b) {
+      const uint32_t e = (uint32_t)((32 * b + n) * HW + 32 * w + 8 * g) * 4;
+      const f32x4 v0 = buf_load16<f32x4>(r, e), v1 = buf_load16<f32x4>(r, e + 16);
+      const f32x4 v2 = buf_load16<f32x4>(r, e + 64), v3 = buf_load16<f32x4>(r, e + 80);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        dst[l][j] = a[j];
-        dst[l][4 + j] = b[j];
-        dst[l][8 + j] = c[j];
-        dst[l][12 + j] = d[j];
+        h[l][b][j] = v0[j];
+        h[l][b][4 + j] = v1[j];
+        h[l][b][8 + j] = v2[j];
+        h[l][b][12 + j] = v3[j];
       }
     }
   }
+  template <int l = L - 1>
+  __device__ __forceinline__ void load_all_h(int64_t row0) {
+    if constexpr (l >= 1) {
+      load_h<l>(row0);
+      load_all_h<l - 1>(row0);
+    }
+  }
 
-  // Stores 16 values of row n (features 32w + 8g + [0..7], 32w + 16 + 8g +
-  // [0..7]) into a [M, W] tensor of the mode's element type; halves past the
-  // true width are dropped.
-  __device__ __forceinline__ void store_row16(void* base, int W, int64_t row0, const float (&v)[16]) const {
-    const rsrc_t r = make_rsrc(static_cast<char*>(base) + row0 * W * kEs<EM>, rows_at(p.M, row0, 32) * W * kEs<EM>);
-    const uint32_t e = (uint32_t)(n * W + 32 * w + 8 * g);
+  // Stores 16 values of row 32b + n (features 32w + 8g + [0..7], 32w + 16 +
+  // 8g + [0..7]) into a [M, W] tensor of the mode's element type; halves past
+  // the true width are dropped.
+  __device__ __forceinline__ void store_row16(rsrc_t r, int W, int b, const float (&v)[16]) const {
+    const uint32_t e = (uint32_t)((32 * b + n) * W + 32 * w + 8 * g);
     if (!N::gen || 32 * w < W) store8<EM>(r, e, v);
     if (!N::gen || 32 * w + 16 < W) store8<EM>(r, e + 16, v + 8);
   }
+  __device__ __forceinline__ rsrc_t rows_rsrc(void* base, int W, int64_t row0) const {
+    return make_rsrc(static_cast<char*>(base) + row0 * W * kEs<EM>, rows_at(p.M, row0, ROWS) * W * kEs<EM>);
+  }
 
-  // Layer l of one 32-row block: B holds dz_l of the rows.  Owning waves
-  // compute their 32 features of dz_{l-1} = (dz_l W_l^T) * sigma(h_l) (or of
-  // dx for l = 0) and store them; the next layer's B operands then come back
-  // from the exchange tile (all of dz_{l-1}, the other waves' features too).
+  // The MFMAs of layer l: acc[b] = W_l rows [32w, + 32) . dz_l of row block b.
   template <int l>
-  __device__ __forceinline__ void layer(int64_t row0) {
-    if constexpr (l >= G::LO) {
-      if (owns(l)) {
-        // Two independent accumulator chains (even and odd K-steps) halve
-        // the dependent MFMA latency of the step.
-        f32x16 acc = {}, acc2 = {};
-        if constexpr (RES) {
+  __device__ __forceinline__ void chain(f32x16 (&acc)[RB], int t) {
+    const f16x8* th = tile[t][0];
+    const f16x8* tl = tile[t][NT - 1];
+    auto read = [&](Opnd (&o)[RB], int s) {
 #pragma unroll
-          for (int s = 0; s < G::ks(l); ++s) {
-            if (s & 1)
-              acc2 = mma<EM>(fr[l][s], B[s], acc2);
-            else
-              acc = mma<EM>(fr[l][s], B[s], acc);
-          }
-        } else {
-          Opnd f[G::KSM];
-          frags_of<l>(f);
-          if constexpr (l >= 1) load_h_one<l>(row0, h);
+      for (int b = 0; b < RB; ++b) {
+        o[b].h = th[slot<CH>(32 * b + n, 2 * s + g)];
+        o[b].l = NT == 2 ? tl[slot<CH>(32 * b + n, 2 * s + g)] : f16x8{};
+      }
+    };
+    Opnd in[2][RB];
+    read(in[0], 0);
+    if constexpr (RES) {
 #pragma unroll
-          for (int s = 0; s < G::ks(l); ++s) {
-            if (s & 1)
-              acc2 = mma<EM>(f[s], B[s], acc2);
-            else
-              acc = mma<EM>(f[s], B[s], acc);
-          }
+      for (int s = 0; s < G::ks(l); ++s) {
+        if (s + 1 < G::ks(l)) read(in[(s + 1) & 1], s + 1);
+#pragma unroll
+        for (int b = 0; b < RB; ++b) acc[b] = mma<EM>(fr[l][s], in[s & 1][b], acc[b]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      // Whole turns of kRing K-steps: the tile holds zeros up to a multiple of
+      // 64 features.
+      const int KS = (dimw<N>(p, l + 1) + 15) / 16;
+      for (int c = 0; c < KS; c += kRing) {
+#pragma unroll
+        for (int t = 0; t < kRing; ++t) {
+          read(in[(t + 1) & 1], c + t + 1 < KS ? c + t + 1 : 0);  // (past the last one: K-step 0 again)
+          const Opnd a = to_op(ring[t]);
+#pragma unroll
+          for (int b = 0; b < RB; ++b) acc[b] = mma<EM>(a, in[t & 1][b], acc[b]);
+          ring[t] = load_frag<l>(c + kRing + t);
+          __builtin_amdgcn_sched_barrier(0);
         }
-        acc += acc2;
-        float v[16];
-        if constexpr (l >= 1) {
+      }
+    }
+  }
+
+  // Layer l of the tile at row0 (the next one at `next`): tile[par] holds dz_l.
+  // Owning waves compute their 32 features of dz_{l-1} = (dz_l W_l^T) *
+  // sigma(h_l) (or of dx for l = 0), store them and hand them on.
+  template <int l>
+  __device__ __forceinline__ void layer(int64_t row0, int64_t next) {
+    constexpr bool HAND = l >= 1 && l - 1 >= G::LO;  // another layer follows
+    f32x16 acc[RB] = {};
+    if (owns(l)) chain<l>(acc, par);
+    request<(HAND ? l - 1 : L - 1)>();
+    par ^= 1;
+    if constexpr (l >= 1) {
+      const int W = dimw<N>(p, l);
+      const rsrc_t dz = rows_rsrc(p.dz[l - 1], W, row0);
 #pragma unroll
-          for (int j = 0; j < 16; ++j) v[j] = acc[j] * sig_from_h(h[l][j]);
-          store_row16(p.dz[l - 1], dimw<N>(p, l), row0, v);  // for the weight-gradient pass
-          if constexpr (l - 1 >= G::LO) {  // and for the next layer, through the tile
+      for (int b = 0; b < RB; ++b) {
+        float v[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) v[j] = acc[b][j] * sig_from_h(h[l][b][j]);
+        store_row16(dz, W, b, v);  // for the weight-gradient pass
+        if constexpr (HAND) {      // and for the next layer, through the tile (waves past the width write zeros)
+          if (!N::gen || 32 * w < ((W + 63) & ~63)) {
             const Opnd lo = make_op<EM>(*reinterpret_cast<const float(*)[8]>(v));
             const Opnd hi = make_op<EM>(*reinterpret_cast<const float(*)[8]>(v + 8));
-            tile[par][0][slot<CH>(n, 4 * w + g)] = lo.h;
-            tile[par][0][slot<CH>(n, 4 * w + 2 + g)] = hi.h;
+            tile[par][0][slot<CH>(32 * b + n, 4 * w + g)] = lo.h;
+            tile[par][0][slot<CH>(32 * b + n, 4 * w + 2 + g)] = hi.h;
             if constexpr (NT == 2) {
-              tile[par][NT - 1][slot<CH>(n, 4 * w + g)] = lo.l;
-              tile[par][NT - 1][slot<CH>(n, 4 * w + 2 + g)] = hi.l;
+              tile[par][NT - 1][slot<CH>(32 * b + n, 4 * w + g)] = lo.l;
+              tile[par][NT - 1][slot<CH>(32 * b + n, 4 * w + 2 + g)] = hi.l;
             }
           }
-        } else {
-#pragma unroll
-          for (int j = 0; j < 16; ++j) v[j] = acc[j];
-          store_row16(p.dx, dimw<N>(p, 0), row0, v);
         }
       }
-      if constexpr (l >= 1 && l - 1 >= G::LO) {
-        __syncthreads();  // the whole of dz_{l-1} of these rows is in the tile
-        const int Wd = dimw<N>(p, l);  // features of dz_{l-1} the waves wrote
+      load_h<l>(next);
+    } else {
+      const int W = dimw<N>(p, 0);
+      const rsrc_t dx = rows_rsrc(p.dx, W, row0);
 #pragma unroll
-        for (int s = 0; s < G::ks(l - 1); ++s) {
-          B[s].h = tile[par][0][slot<CH>(n, 2 * s + g)];
-          B[s].l = NT == 2 ? tile[par][NT - 1][slot<CH>(n, 2 * s + g)] : f16x8{};
-          // Past the true width the tile holds whatever an earlier block
-          // left there (or nothing): zero operands, so that it cannot meet
-          // the zero fragments as inf * 0 = NaN.
-          if (N::gen && 16 * s + 8 * g >= Wd) B[s] = Opnd{f16x8{}, f16x8{}};
-        }
-        // The next hand-over writes the other tile: this one is read until
-        // every wave has passed the next barrier.
-        par ^= 1;
-        layer<l - 1>(row0);
+      for (int b = 0; b < RB; ++b) {
+        float v[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) v[j] = acc[b][j];
+        if (owns(0)) store_row16(dx, W, b, v);
       }
+    }
+    if constexpr (HAND) {
+      // The whole of dz_{l-1} of these rows is in the tile.  (The other tile,
+      // read just now, is written after this barrier at the earliest.)
+      __syncthreads();
+      layer<l - 1>(row0, next);
     }
   }
 };
 
-template <class N, int EM, bool DX, bool RES>
+template <class N, int EM, bool DX, bool RES, int RB>
 __global__ __launch_bounds__((DgGeo<N, DX>::NWV * 64)) void tp_dgrad_kernel(TpParams p) {
   using G = DgGeo<N, DX>;
-  using W = DgWave<N, EM, DX, RES>;
+  using W = DgWave<N, EM, DX, RES, RB>;
   static_assert(G::valid(), "two-pass backward shape");
-  __shared__ f16x8 tile[2][W::NT][32 * G::CH];  // two exchange tiles (hi, and lo with fp32 tensors)
+  __shared__ f16x8 tile[2][W::NT][W::ROWS * G::CH];  // two exchange tiles (hi, and lo with fp32 tensors)
   const int lane = threadIdx.x & 63;
-  __shared__ f16x8 stage[W::STG_ELEMS];  // STG: one layer's fragments
   W wv{p, tile, lane, lane & 31, lane >> 5, __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))};
-  if constexpr (W::STG) {
-    wv.stg = stage;
-    wv.stage_largest();  // (each wave reads back only what it wrote: no barrier)
-  }
-  const int64_t nblk = (p.M + 31) / 32;
+  const int64_t ntiles = (p.M + W::ROWS - 1) / W::ROWS;
   if (p.zero_dw) {
     // Written (=) rather than accumulated dW: cleared here, before the
     // weight-gradient pass adds its tiles (the next launch on the stream).
@@ -380,18 +383,17 @@ __global__ __launch_bounds__((DgGeo<N, DX>::NWV * 64)) void tp_dgrad_kernel(TpPa
       for (int64_t i = tid; i < n4; i += nthr) d[i] = f32x4{};
     }
   }
-  if constexpr (RES) {
-    wv.template load_h<>((int64_t)blockIdx.x * 32, wv.hn);  // (from HBM: the longest wait first)
-    wv.template load_all_frags<>();                          // (L2 hits after the first workgroup)
-  }
-  for (int64_t b = blockIdx.x; b < nblk; b += gridDim.x) {
-    const int64_t row0 = b * 32;
-    if constexpr (RES) {
-      wv.take_next_h();
-      wv.template load_h<>(row0 + 32 * (int64_t)gridDim.x, wv.hn);
-    }
-    wv.load_dout(row0);
-    wv.template layer<N::L - 1>(row0);
+  int64_t t = blockIdx.x;
+  wv.load_dout(t * W::ROWS);
+  wv.template load_all_h<>(t * W::ROWS);  // (from HBM: the longest wait first)
+  if constexpr (RES) wv.template load_all_frags<>();  // (L2 hits after the first workgroup)
+  wv.template request<N::L - 1>();
+  for (; t < ntiles; t += gridDim.x) {
+    const int64_t row0 = t * W::ROWS, next = row0 + (int64_t)gridDim.x * W::ROWS;
+    wv.commit_dout();
+    wv.load_dout(next);
+    __syncthreads();  // dL/dout of these rows is in the tile
+    wv.template layer<N::L - 1>(row0, next);
   }
 }
 
@@ -689,20 +691,27 @@ int cached_occupancy(const void* kern, int threads, int* occ_out) {
   return MLPMK_OK;
 }
 
-template <class N, int EM, bool DX, bool RES>
-int launch_dgrad(const TpParams& p, int cus, hipStream_t st) {
+template <class N, int EM, bool DX, bool RES, int RB>
+int launch_dgrad_rb(const TpParams& p, int cus, hipStream_t st) {
   using G = tp::DgGeo<N, DX>;
-  const void* kern = reinterpret_cast<const void*>(&tp::tp_dgrad_kernel<N, EM, DX, RES>);
+  const void* kern = reinterpret_cast<const void*>(&tp::tp_dgrad_kernel<N, EM, DX, RES, RB>);
   int occ = 0;
   int rc = cached_occupancy(kern, G::NWV * 64, &occ);
   if (rc != MLPMK_OK) return rc;
-  const int64_t nblk = (p.M + 31) / 32;
+  const int64_t ntiles = (p.M + 32 * RB - 1) / (32 * RB);
   const int64_t cap = (int64_t)cus * occ;
-  const int grid = (int)(nblk < cap ? nblk : cap);
+  const int grid = (int)(ntiles < cap ? ntiles : cap);
   (void)hipGetLastError();
-  hipLaunchKernelGGL((tp::tp_dgrad_kernel<N, EM, DX, RES>), dim3(grid), dim3(G::NWV * 64), 0, st, p);
+  hipLaunchKernelGGL((tp::tp_dgrad_kernel<N, EM, DX, RES, RB>), dim3(grid), dim3(G::NWV * 64), 0, st, p);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? MLPMK_OK : hip_fail(e, "two-pass dgrad kernel launch");
+}
+
+// Tiles of 64 rows where that still gives every CU one, else of 32 rows.
+template <class N, int EM, bool DX, bool RES>
+int launch_dgrad(const TpParams& p, int cus, hipStream_t st) {
+  return p.M > (int64_t)64 * cus ? launch_dgrad_rb<N, EM, DX, RES, 2>(p, cus, st)
+                                 : launch_dgrad_rb<N, EM, DX, RES, 1>(p, cus, st);
 }
 
 // Weight-gradient tiling: a workgroup owns TQ x TQ quads (64 x 64 blocks of
