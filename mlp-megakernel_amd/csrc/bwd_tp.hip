@@ -26,34 +26,33 @@
 //     dz_{l-1} = (dz_l . W_l^T) * (1 - exp(-h_l)),   dx = dz_0 . W_0^T
 //     dW_l     = a_l^T . dz_l
 //
-// Pass 1, tp_dgrad_kernel (persistent over 32-row blocks, one workgroup per
-// block at a time): wave w owns output features [32w, 32w + 32) of every
-// data-gradient layer, with its A fragments (16 contiguous bytes of a W_l
-// row per lane) loaded once into registers for the 3-layer 128-wide network
-// -- which then loads the next block's stash rows while the current block
-// computes -- and read from L2 per block and layer otherwise; layers hand dz
-// between waves through two LDS tiles, and every dz_{l-1}, l >= 1, is also
-// written to the workspace.  When dw is to be written (MLPMK_BWD_WRITE_DW)
-// this pass also clears it.  At M = 4096 that is 128 workgroups each running
-// a chain of 8-MFMA steps, instead of 32 running whole 128-row rounds.
+// Pass 1, tp_dgrad_kernel (persistent over tiles of 32 or 64 rows): wave w owns
+// output features [32w, 32w + 32) of every data-gradient layer, with its A
+// fragments (16 contiguous bytes of a W_l row per lane) loaded once into
+// registers for the 3-layer 128-wide network and read from L2 otherwise;
+// layers hand dz between waves through two LDS tiles, and every dz_{l-1},
+// l >= 1, is also written to the workspace.  The next tile's rows are
+// requested while this one computes.  When dw is to be written
+// (MLPMK_BWD_WRITE_DW) this pass also clears it.  At M = 4096 that is 128
+// workgroups each running a chain of 8-MFMA steps, instead of 32 running
+// whole 128-row rounds.
 //
 // Pass 2, tp_wgrad_kernel: a workgroup owns a TQI x TQO block of 64 x 64
 // "quads" of one dW_l and a chunk of rows; it stages a_l (from x or the
-// stash) and dz_l (from dL/dout or the workspace), 64 KiB of rows at a time,
-// as 16-bit tiles [row][feature] in LDS, and its waves read both MFMA
-// operands with the transposing ds_read_b64_tr_b16, as bwd.hip's wgrad does.
-// Each wave adds its 32 x 32 tiles to dw with fp32 atomics: about two
-// workgroups per CU (with a register budget that lets both stay resident
-// when the grid exceeds the CU count), each adding 4096 elements, so the
-// atomics are spread over the whole chip (measured at M = 4096 / 16384: 14.2 / 24.1 us per
-// backward, against 16.4 / 31.0 us with per-chunk partial sums and a
-// combine kernel).  The summation order of dw is therefore not fixed.
+// stash) and dz_l (from dL/dout or the workspace) as 16-bit tiles
+// [row][feature] in LDS, and its waves read both MFMA operands with the
+// transposing ds_read_b64_tr_b16, as bwd.hip's wgrad does.  Its sums go to dw
+// as fp32 atomics at the end (measured at M = 4096 / 16384: 14.2 / 24.1 us per
+// backward, against 16.4 / 31.0 us with per-chunk partial sums and a combine
+// kernel).  The summation order of dw is therefore not fixed.
 //
 // Where it runs (bwd.hip, bwd_path): fp32 tensors and widths above 128
 // always; the 16-bit networks the one-pass megakernel also serves up to
 // MLPMK_TP_MAX_ROWS rows (3L-128, MI355X, per backward call as a replayed
 // graph, two-pass vs one-pass: 14.2 vs 23.0 us at 4096 rows, 24.1 vs 26.8 at
 // 16384, 42.6 vs 33.3 at 32768).
+#include <type_traits>
+
 #include "device_common.h"
 #include "host_common.h"
 #include "params.h"
@@ -401,46 +400,53 @@ __global__ __launch_bounds__((DgGeo<N, DX>::NWV * 64)) void tp_dgrad_kernel(TpPa
 // Pass 2: weight gradients
 // ---------------------------------------------------------------------------
 
-// A workgroup of 4 waves owns TQI x TQO quads (64 x 64 blocks of dW_l): its
-// LDS tile rows hold 64 TQI features of a_l and then 64 TQO features of dz_l,
-// RP rows per pass (64 KiB of tiles).  With one quad each wave owns one of
-// its four 32 x 32 tiles; with four quads, each wave one quad.  Every wave
-// runs all the K-rows of the pass for its tiles, so no partial sums meet
-// across waves.
-template <int EM, int TQI, int TQO>
+// A workgroup owns TQI x TQO quads (64 x 64 blocks of dW_l): its LDS tile rows
+// hold 64 TQI features of a_l and then 64 TQO features of dz_l, RP rows per
+// pass.  With one quad its four waves own one 32 x 32 tile each; otherwise a
+// wave owns a quad.  Every wave runs all the K-rows of a pass for its tiles.
+// KG wave groups (each with its own LDS tile) take the chunk's passes in
+// turns and add up through LDS at the end: the rows in flight of that many
+// workgroups, for the atomics of one.
+template <int EM, int TQI, int TQO, int KG>
 struct WgGeo {
   static constexpr int QW = TQI * TQO;
-  static constexpr int TPW = QW;                     // 32 x 32 tiles per wave
+  static constexpr int GW = QW == 1 ? 4 : QW;        // waves per group
+  static constexpr int GT = 64 * GW, THREADS = KG * GT;
+  static constexpr int TPW = QW == 1 ? 1 : 4;        // 32 x 32 tiles per wave
   static constexpr int FA = 64 * TQI, FZ = 64 * TQO, F = FA + FZ;
   static constexpr int NT = EM == EM_F32 ? 2 : 1;    // tiles: hi (and lo)
-  static constexpr int RP = 32768 / F / NT;          // rows per pass
-  static constexpr int PA = RP * FA / 8 / 256;       // 8-element pieces of a_l per thread per pass
-  static constexpr int PZ = RP * FZ / 8 / 256;       // and of dz_l
+  static constexpr int RP = F > 256 ? 128 : 32768 / F / NT;  // rows per pass
+  static constexpr int PA = RP * FA / 8 / GT;        // 8-element pieces of a_l per thread per pass
+  static constexpr int PZ = RP * FZ / 8 / GT;        // and of dz_l
   static constexpr int KS = RP / 16;                 // K-steps per pass
-  static constexpr int LDS_BYTES = NT * RP * F * 2;
-  static_assert(QW == 1 || QW == 4, "one quad per workgroup or one per wave");
+  static constexpr int TILE = NT * RP * F;           // 16-bit elements of a group's tiles
+  static constexpr int LDS_BYTES = KG * TILE * 2;
+  static_assert(QW == 1 || QW == 4 || (QW == 8 && EM != EM_F32), "one quad per workgroup or one per wave");
+  static_assert(KG == 1 || (KG == 2 && QW == 4 && LDS_BYTES >= 2 * GW * 2 * 4096), "the groups' sums meet in the tiles");
 };
 
 // Tile layout: element (r, f) of a tile with F features per row sits at
-// r*F + (f ^ swz(r, F)); the XOR moves whole 8-feature chunks, so 16-byte
+// r*F + (f ^ swz(r, F)), where F is a power of two (else each half of the row
+// for itself); the XOR moves whole 8-feature chunks, so 16-byte
 // writes and 8-byte transposed reads stay contiguous, and the four rows of
 // one transposed read land in four distinct 16-feature windows.
 __device__ __forceinline__ int swz(int r, int F) {
   return (16 * (r & 3) + 8 * ((r >> 2) & 1) + 64 * ((r >> 3) & 1)) & (F - 1);
 }
 
-// MFMA operand for features fb .. fb+31 over rows 16kk .. 16kk+15 of a tile:
+// MFMA operand for features fb .. fb+31 over rows 16kk .. 16kk+15 of a tile of
+// F features a row (F0, FS: first feature and extent of the XOR):
 // lane (m, g) gets rows 16kk + 8g + [0..7] of feature fb + m, through two
 // transposing reads (per 16-lane group: result lane i, element j is element
 // i & 3 of the 8 bytes addressed by lane (i >> 2) + 4j).
-template <int F>
+template <int F, int F0, int FS>
 __device__ __forceinline__ f16x8 xread(const f16* t, int fb, int kk, const int (&rrow)[2], int rcol) {
   typedef short s16x4 __attribute__((ext_vector_type(4)));
   s16x4 h[2];
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
     const int r = rrow[k];
-    const f16* a = t + (16 * kk + r) * F + ((fb + rcol) ^ swz(r, F));
+    const f16* a = t + (16 * kk + r) * F + F0 + ((fb + rcol) ^ swz(r, FS));
     h[k] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)const_cast<f16*>(a));
   }
   return __builtin_bit_cast(f16x8, __builtin_shufflevector(h[0], h[1], 0, 1, 2, 3, 4, 5, 6, 7));
@@ -457,19 +463,17 @@ struct WgSrc {
   uint32_t bytes;    // resource size from base
 };
 
-// MINW: waves per SIMD the register allocation must leave room for.  2 when
-// the grid has more workgroups than CUs: two workgroups per CU then keep
-// twice the rows in flight (fp32 3L-128 at 131072 rows 228 -> 217 us,
-// 128-256-256-128 400 -> 373 us per backward; the 128x128 blocks need 222-228
-// VGPRs + 64 AGPRs left to themselves, one workgroup per CU).  1 for grids of
-// at most one workgroup per CU (128-256-256-128 at 4096 rows: 38.2 us, 40.7
-// with the tighter budget).
-template <class N, int EM, int TQI, int TQO, int MINW>
-__global__ __launch_bounds__(256, MINW) void tp_wgrad_kernel(TpParams p) {
-  using G = WgGeo<EM, TQI, TQO>;
-  constexpr int F = G::F, RP = G::RP, NT = G::NT;
+// MINW: waves per SIMD the register allocation must leave room for: 2 for the
+// 4-wave kernels when the grid has more workgroups than CUs (two workgroups
+// per CU keep twice the rows in flight).
+template <class N, int EM, int TQI, int TQO, int KG, int MINW>
+__global__ __launch_bounds__((WgGeo<EM, TQI, TQO, KG>::THREADS), MINW) void tp_wgrad_kernel(TpParams p) {
+  using G = WgGeo<EM, TQI, TQO, KG>;
+  constexpr int F = G::F, RP = G::RP, NT = G::NT, GT = G::GT;
+  constexpr bool kPow2 = (F & (F - 1)) == 0;
   __shared__ __attribute__((aligned(16))) char smem[G::LDS_BYTES];
-  f16* const tiles = reinterpret_cast<f16*>(smem);
+  const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / GT);  // this wave's group
+  f16* const tiles = reinterpret_cast<f16*>(smem) + kg * G::TILE;
   const int L = N::L;
   // Task: (layer, quad block) from blockIdx.y, row chunk from blockIdx.x.
   int l = 0, bi = 0, bo = 0;
@@ -487,8 +491,10 @@ __global__ __launch_bounds__(256, MINW) void tp_wgrad_kernel(TpParams p) {
     }
   }
   const int K = dimw<N>(p, l), NO = dimw<N>(p, l + 1);
-  const int64_t r_begin = (int64_t)blockIdx.x * p.chunk_rows;
-  const int64_t r_end = r_begin + p.chunk_rows < p.M ? r_begin + p.chunk_rows : p.M;
+  const int64_t passes = (p.M + RP - 1) / RP;  // split evenly over the chunks
+  const int64_t r_begin = passes * blockIdx.x / gridDim.x * RP;
+  const int64_t r_next = passes * (blockIdx.x + 1) / gridDim.x * RP;
+  const int64_t r_end = r_next < p.M ? r_next : p.M;
   const int64_t nrows = r_end - r_begin;
   // Sources.  Resources clip to the chunk's rows, so loads past them read 0.
   WgSrc sa, sz;
@@ -517,32 +523,38 @@ __global__ __launch_bounds__(256, MINW) void tp_wgrad_kernel(TpParams p) {
     }
   }
   const rsrc_t ra = make_rsrc(sa.base, sa.bytes), rz = make_rsrc(sz.base, sz.bytes);
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = (int)threadIdx.x - kg * GT, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   // Loads of one pass.  a_l pieces first (8 features each), then dz_l
-  // pieces: piece k of this thread is q = tid + 256 k, row q / (FA / 8)
+  // pieces: piece k of this thread is q = tid + GT k, row q / (FA / 8)
   // (resp. FZ / 8), chunk q % (FA / 8) -- consecutive threads read
   // consecutive 16-byte pieces of a row.  Raw payloads: up to 32 bytes (8
-  // fp32) per piece, kept until the tile is free.
+  // fp32) per piece, kept until the tile is free (16-bit dz: 16 bytes).
   struct Raw {
     f32x4 a, b;
   };
-  Raw raw_a[G::PA], raw_z[G::PZ];
+  struct Raw16 {
+    f32x4 a;
+  };
+  Raw raw_a[G::PA];
+  typename std::conditional<EM == EM_F32, Raw, Raw16>::type raw_z[G::PZ];
   auto issue_src = [&](auto& raw, const WgSrc& s, rsrc_t rr, int FS, int64_t prow) {
     constexpr int NP = sizeof(raw) / sizeof(raw[0]);
+    constexpr bool WIDE = sizeof(raw[0]) > 16;  // the piece may be fp32
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-      const int q = tid + 256 * k, r = q / (FS / 8), c = q % (FS / 8);
+      const int q = tid + GT * k, r = q / (FS / 8), c = q % (FS / 8);
       const int f = s.f0 + 8 * c;
       const int64_t row = prow + r;
       const bool ok = f < s.width && row < nrows;
       const int64_t e = s.stride < 0 ? 0 : row * s.stride + f;
-      raw[k].a = raw[k].b = f32x4{};
+      raw[k].a = f32x4{};
+      if constexpr (WIDE) raw[k].b = f32x4{};
       if (!ok) continue;
-      if (s.es == 4) {
+      if (WIDE && s.es == 4) {
         raw[k].a = buf_load16<f32x4>(rr, (uint32_t)(e * 4));
-        raw[k].b = buf_load16<f32x4>(rr, (uint32_t)(e * 4 + 16));
+        if constexpr (WIDE) raw[k].b = buf_load16<f32x4>(rr, (uint32_t)(e * 4 + 16));
       } else if (s.stride < 0) {  // one 16-bit element for every row and feature
         const int v = __builtin_amdgcn_raw_buffer_load_b16(rr, 0, 0, 0);
         const int vv = (v & 0xffff) | (v << 16);
@@ -560,23 +572,25 @@ __global__ __launch_bounds__(256, MINW) void tp_wgrad_kernel(TpParams p) {
   // features [0, FA), dz_l at [FA, F) of each tile row.
   auto commit_src = [&](const auto& raw, const WgSrc& s, int FS, int fbase) {
     constexpr int NP = sizeof(raw) / sizeof(raw[0]);
+    constexpr bool WIDE = sizeof(raw[0]) > 16;
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-      const int q = tid + 256 * k, r = q / (FS / 8), c = q % (FS / 8);
+      const int q = tid + GT * k, r = q / (FS / 8), c = q % (FS / 8);
       Opnd o;
-      if (s.es == 4) {
-        float v[8] = {raw[k].a[0], raw[k].a[1], raw[k].a[2], raw[k].a[3],
-                      raw[k].b[0], raw[k].b[1], raw[k].b[2], raw[k].b[3]};
-        if (s.stride < 0) {  // (fp32 scalar: element 0 everywhere)
+      o.h = __builtin_bit_cast(f16x8, raw[k].a);
+      o.l = f16x8{};
+      if constexpr (WIDE) {
+        if (s.es == 4) {
+          float v[8] = {raw[k].a[0], raw[k].a[1], raw[k].a[2], raw[k].a[3],
+                        raw[k].b[0], raw[k].b[1], raw[k].b[2], raw[k].b[3]};
+          if (s.stride < 0) {  // (fp32 scalar: element 0 everywhere)
 #pragma unroll
-          for (int j = 1; j < 8; ++j) v[j] = v[0];
+            for (int j = 1; j < 8; ++j) v[j] = v[0];
+          }
+          o = make_op<EM>(v);
         }
-        o = make_op<EM>(v);
-      } else {
-        o.h = __builtin_bit_cast(f16x8, raw[k].a);
-        o.l = f16x8{};
       }
-      const int off = r * F + ((fbase + 8 * c) ^ swz(r, F));
+      const int off = r * F + (kPow2 ? (fbase + 8 * c) ^ swz(r, F) : fbase + ((8 * c) ^ swz(r, FS)));
       *reinterpret_cast<f16x8*>(tiles + off) = o.h;
       if constexpr (NT == 2) *reinterpret_cast<f16x8*>(tiles + RP * F + off) = o.l;
     }
@@ -597,33 +611,61 @@ __global__ __launch_bounds__(256, MINW) void tp_wgrad_kernel(TpParams p) {
     rcol = 16 * (q & 1) + 4 * (i & 3);
   }
   f32x16 acc[G::TPW] = {};
-  auto opnd = [&](int fb, int kk) {
+  auto opnd_a = [&](int fb, int kk) {
+    constexpr int FS = kPow2 ? F : G::FA;
     Opnd o;
-    o.h = xread<F>(tiles, fb, kk, rrow, rcol);
-    o.l = NT == 2 ? xread<F>(tiles + RP * F, fb, kk, rrow, rcol) : f16x8{};
+    o.h = xread<F, 0, FS>(tiles, fb, kk, rrow, rcol);
+    o.l = NT == 2 ? xread<F, 0, FS>(tiles + RP * F, fb, kk, rrow, rcol) : f16x8{};
+    return o;
+  };
+  auto opnd_z = [&](int fb, int kk) {
+    constexpr int F0 = kPow2 ? 0 : G::FA, FS = kPow2 ? F : G::FZ;
+    Opnd o;
+    o.h = xread<F, F0, FS>(tiles, (kPow2 ? G::FA : 0) + fb, kk, rrow, rcol);
+    o.l = NT == 2 ? xread<F, F0, FS>(tiles + RP * F, (kPow2 ? G::FA : 0) + fb, kk, rrow, rcol) : f16x8{};
     return o;
   };
   const int npass = (int)((nrows + RP - 1) / RP);
-  issue(0);
-  for (int ps = 0; ps < npass; ++ps) {
+  // (A group's turn past the last pass reads nothing and adds zeros: every
+  // wave runs the same barriers.)
+  issue((int64_t)kg * RP);
+  for (int ps = kg; ps - kg < npass; ps += KG) {
     __syncthreads();  // the previous pass's reads are done
     commit();
-    if (ps + 1 < npass) issue((int64_t)(ps + 1) * RP);
+    if (ps - kg + KG < npass) issue((int64_t)(ps + KG) * RP);
     __syncthreads();  // the tile is written
     // (K-steps past the chunk's last row read zeros: the loads were masked.)
 #pragma unroll
     for (int kk = 0; kk < G::KS; ++kk) {
       if constexpr (G::QW == 1) {
-        acc[0] = mma<EM>(opnd(32 * (w >> 1), kk), opnd(G::FA + 32 * (w & 1), kk), acc[0]);
+        acc[0] = mma<EM>(opnd_a(32 * (w >> 1), kk), opnd_z(32 * (w & 1), kk), acc[0]);
       } else {
-        const Opnd a0 = opnd(64 * qi, kk), a1 = opnd(64 * qi + 32, kk);
-        const Opnd b0 = opnd(G::FA + 64 * qo, kk), b1 = opnd(G::FA + 64 * qo + 32, kk);
+        const Opnd a0 = opnd_a(64 * qi, kk), a1 = opnd_a(64 * qi + 32, kk);
+        const Opnd b0 = opnd_z(64 * qo, kk), b1 = opnd_z(64 * qo + 32, kk);
         acc[0] = mma<EM>(a0, b0, acc[0]);
         acc[1] = mma<EM>(a0, b1, acc[1]);
         acc[2] = mma<EM>(a1, b0, acc[2]);
         acc[3] = mma<EM>(a1, b1, acc[3]);
       }
     }
+  }
+  if constexpr (KG == 2) {
+    // Group 0 takes tiles 0 and 1 of every quad, group 1 tiles 2 and 3: each
+    // leaves the other's two in LDS.
+    float* const sum = reinterpret_cast<float*>(smem) + w * 2048 + lane;
+    __syncthreads();  // the last pass's reads are done
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) sum[kg * G::GW * 2048 + t * 1024 + e * 64] = kg ? acc[t][e] : acc[2 + t][e];
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const float v = sum[(1 - kg) * G::GW * 2048 + t * 1024 + e * 64];
+        acc[t][e] = (kg ? acc[2 + t][e] : acc[t][e]) + v;
+      }
   }
 
   // Output: tile t = 2 ti + to of quad (qi, qo): C lane (o, g), register e
@@ -642,6 +684,9 @@ __global__ __launch_bounds__(256, MINW) void tp_wgrad_kernel(TpParams p) {
   };
   if constexpr (G::QW == 1) {
     write_tile(acc[0], w);
+  } else if constexpr (KG == 2) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) write_tile(acc[t], 2 * kg + t);
   } else {
 #pragma unroll
     for (int t = 0; t < 4; ++t) write_tile(acc[t], t);
@@ -714,25 +759,35 @@ int launch_dgrad(const TpParams& p, int cus, hipStream_t st) {
                                  : launch_dgrad_rb<N, EM, DX, RES, 1>(p, cus, st);
 }
 
-// Weight-gradient tiling: a workgroup owns TQ x TQ quads (64 x 64 blocks of
-// dW).  One quad per workgroup (TQ = 1) gives small batches enough
-// workgroups; four (TQ = 2) read each a_l and dz_l element fewer times.
-int wgrad_tq(int L, const int* dims, int64_t M) {
+// Weight-gradient tiling (WgGeo): WG_QUAD, one 64 x 64 block per 4-wave
+// workgroup, gives small batches enough workgroups; the others read each a_l
+// and dz_l element fewer times.  WG_PAIR: 128 x 128 blocks, 8 waves in two
+// groups (widths up to 128: each operand read once).  WG_WIDE: 128 x 256
+// blocks, 8 waves (16-bit tensors of widths above 128: the fp32 activations
+// read once, dz twice).
+//
+// Where the lines lie (this pass alone, us; QUAD / the other form):
+// 128-256-256-128 bf16 at 4,096 rows 11 / 23, 16,384 23 / 33, 32,768 39 / 45,
+// 49,152 54 / 52, 100,003 155 / 91 (4-wave 128 x 128 blocks, which WG_WIDE
+// replaced: 19, 41, 46, 53, 113); 160-192-192-192-64 fp16 at 49,152 89 / 55.
+// 3x128 fp32 at 16,384 23 / 30, 32,768 35 / 34, 49,152 50 / 43 (4-wave 128 x
+// 128 at 65,536: 60, WG_PAIR 46: half the atomics, 23 us of the 60).  Below 64
+// features a 128 x 128 block is mostly empty: 3x64 fp32 32 / 32 at 65,536.
+enum { WG_QUAD, WG_PAIR, WG_WIDE };
+constexpr int kPairMinRows = 32768, kWideMinRows = 24576;
+int wgrad_form(int L, const int* dims, int64_t M) {
   int wmax = 0;
   for (int i = 0; i <= L; ++i) wmax = dims[i] > wmax ? dims[i] : wmax;
-  return (wmax > 128 || M >= 65536) ? 2 : 1;
+  if (wmax > 128) return M >= kWideMinRows ? WG_WIDE : WG_QUAD;
+  return wmax > 64 && M >= kPairMinRows ? WG_PAIR : WG_QUAD;
 }
 
-int quad_blocks(int L, const int* dims, int tq) {
-  int nqb = 0;
-  for (int l = 0; l < L; ++l) nqb += ((dims[l] + 64 * tq - 1) / (64 * tq)) * ((dims[l + 1] + 64 * tq - 1) / (64 * tq));
-  return nqb;
+int quad_blocks(int L, const int* dims, int form) {
+  const int fa = form == WG_QUAD ? 64 : 128, fz = form == WG_QUAD ? 64 : form == WG_PAIR ? 128 : 256;
+  int n = 0;
+  for (int l = 0; l < L; ++l) n += ((dims[l] + fa - 1) / fa) * ((dims[l + 1] + fz - 1) / fz);
+  return n;
 }
-
-// Workgroups per CU the weight-gradient grid aims at.
-#ifndef MLPMK_TP_WG_PER_CU
-#define MLPMK_TP_WG_PER_CU 2
-#endif
 
 // Longest row chunk with fp32 tensors.  A chunk's products of split
 // operands accumulate in one MFMA chain per tile, three MFMAs per K-step, and
@@ -744,31 +799,42 @@ int quad_blocks(int L, const int* dims, int tq) {
 // (more atomics) instead.
 constexpr int64_t kF32MaxChunkRows = 8192;
 
-// Row chunks of the weight-gradient pass: enough chunks for about
-// MLPMK_TP_WG_PER_CU workgroups per CU, each a whole number of passes (with
-// fp32 tensors, at most kF32MaxChunkRows rows).
-void wgrad_chunks(int L, const int* dims, int64_t M, bool f32, int cus, int* S_out, int64_t* rows_out) {
-  const int tq = wgrad_tq(L, dims, M);
-  const int rp = (tq == 1 ? 256 : 128) / (f32 ? 2 : 1);  // rows per pass (WgGeo::RP)
-  const int nqb = quad_blocks(L, dims, tq);
-  int64_t smax = ((int64_t)MLPMK_TP_WG_PER_CU * cus + nqb - 1) / nqb;
-  if (smax < 1) smax = 1;
-  int64_t rows = (M + smax - 1) / smax;
-  rows = (rows + rp - 1) / rp * rp;
-  if (f32 && rows > kF32MaxChunkRows) rows = kF32MaxChunkRows;  // a multiple of every rp
-  *rows_out = rows;
-  *S_out = (int)((M + rows - 1) / rows);
+// Row chunks of the weight-gradient pass: as many as let every workgroup run
+// at once (two 4-wave workgroups per CU, one of 8 waves; one more would run
+// after the others), each a whole number of passes -- the fewest chunks that
+// keep the longest one as short while chunks are a few passes long, else that
+// many chunks with the passes spread evenly -- and with fp32 tensors of at
+// most kF32MaxChunkRows rows.
+int wgrad_chunks(int L, const int* dims, int64_t M, bool f32, int cus) {
+  const int form = wgrad_form(L, dims, M);
+  const int rp = (form == WG_QUAD ? 256 : 128) / (f32 ? 2 : 1);  // rows per pass (WgGeo::RP)
+  const int nqb = quad_blocks(L, dims, form);
+  const int64_t passes = (M + rp - 1) / rp;
+  int64_t S = (int64_t)(form == WG_QUAD ? 2 : 1) * cus / nqb;
+  if (S < 1) S = 1;
+  const int64_t longest = (passes + S - 1) / S;
+  if (longest < 4) S = (passes + longest - 1) / longest;
+  if (f32 && S * (kF32MaxChunkRows / rp) < passes) S = (passes + kF32MaxChunkRows / rp - 1) / (kF32MaxChunkRows / rp);
+  return (int)S;
 }
 
-template <class N, int EM, int TQ>
-int launch_wgrad(const TpParams& p, int S, int nqb, int cus, hipStream_t st) {
+template <class N, int EM, int TQI, int TQO, int KG, int MINW>
+int launch_wgrad(const TpParams& p, int S, int nqb, hipStream_t st) {
   (void)hipGetLastError();
-  if ((int64_t)S * nqb > cus)
-    hipLaunchKernelGGL((tp::tp_wgrad_kernel<N, EM, TQ, TQ, 2>), dim3(S, nqb), dim3(256), 0, st, p);
-  else
-    hipLaunchKernelGGL((tp::tp_wgrad_kernel<N, EM, TQ, TQ, 1>), dim3(S, nqb), dim3(256), 0, st, p);
+  hipLaunchKernelGGL((tp::tp_wgrad_kernel<N, EM, TQI, TQO, KG, MINW>), dim3(S, nqb),
+                     dim3(tp::WgGeo<EM, TQI, TQO, KG>::THREADS), 0, st, p);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? MLPMK_OK : hip_fail(e, "two-pass wgrad kernel launch");
+}
+
+template <class N, int EM>
+int launch_wgrad_form(const TpParams& p, int form, int S, int nqb, int cus, hipStream_t st) {
+  if constexpr (EM != tp::EM_F32) {
+    if (form == WG_WIDE) return launch_wgrad<N, EM, 2, 4, 1, 1>(p, S, nqb, st);
+  }
+  if (form == WG_PAIR) return launch_wgrad<N, EM, 2, 2, 2, 1>(p, S, nqb, st);
+  return (int64_t)S * nqb > cus ? launch_wgrad<N, EM, 1, 1, 1, 2>(p, S, nqb, st)
+                                : launch_wgrad<N, EM, 1, 1, 1, 1>(p, S, nqb, st);
 }
 
 int64_t round256(int64_t b) { return (b + 255) / 256 * 256; }
@@ -820,14 +886,11 @@ int dispatch_l(const TpParams& p, const int* dims, int S, hipStream_t st) {
   if (rc != MLPMK_OK) return rc;
   // Pass 2 (the kernel reads only N's layer count and whether its widths are
   // fixed: one runtime-width instance per depth serves every shape).
-  const int tq = wgrad_tq(L, dims, p.M);
-  const int nqb = quad_blocks(L, dims, tq);
+  const int form = wgrad_form(L, dims, p.M);
+  const int nqb = quad_blocks(L, dims, form);
   typedef typename GenTp<L>::W NW;
-  if (L == 3 && is_3l128(L, dims))
-    rc = tq == 1 ? launch_wgrad<TNet3L128, EM, 1>(p, S, nqb, cus, st)
-                 : launch_wgrad<TNet3L128, EM, 2>(p, S, nqb, cus, st);
-  else
-    rc = tq == 1 ? launch_wgrad<NW, EM, 1>(p, S, nqb, cus, st) : launch_wgrad<NW, EM, 2>(p, S, nqb, cus, st);
+  rc = L == 3 && is_3l128(L, dims) ? launch_wgrad_form<TNet3L128, EM>(p, form, S, nqb, cus, st)
+                                   : launch_wgrad_form<NW, EM>(p, form, S, nqb, cus, st);
   return rc;
 }
 
@@ -879,8 +942,7 @@ int tp_dispatch(int L, const int* dims, int dtype, const BwdParams& bp, void* ws
     p.dz[l] = c;
     c += round256(bp.M * dims[l + 1] * es);
   }
-  int S = 0;
-  wgrad_chunks(L, dims, bp.M, dtype == MLPMK_DTYPE_F32, cus, &S, &p.chunk_rows);
+  const int S = wgrad_chunks(L, dims, bp.M, dtype == MLPMK_DTYPE_F32, cus);
   const int em = dtype == MLPMK_DTYPE_F32 ? tp::EM_F32 : dtype == MLPMK_DTYPE_BF16 ? tp::EM_BF16 : tp::EM_F16;
   switch (em * 8 + L) {
 #define MLPMK_TP_CASE(E, LL) \

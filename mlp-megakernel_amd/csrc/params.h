@@ -62,7 +62,6 @@ struct TpParams {
   float* dw[kMaxLayersHost];           // fp32 [d[l], d[l+1]], accumulated into (fp32 atomics)
   void* dz[kMaxLayersHost];            // dz_l, l = 0 .. L-2: [M, d[l+1]] in the workspace
   int64_t M;
-  int64_t chunk_rows;                  // rows per weight-gradient chunk
   // Nonzero: the data-gradient pass clears dw before the weight-gradient
   // pass adds to it (MLPMK_BWD_WRITE_DW).
   int zero_dw;

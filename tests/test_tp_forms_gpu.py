@@ -1,0 +1,57 @@
+"""The two-pass backward (csrc/bwd_tp.hip) at the sizes where its kernels
+change form: data-gradient tiles of 32 and 64 rows, weight-gradient blocks of
+64 x 64 (4 waves), 128 x 128 (two groups of 4 waves that add up through LDS)
+and 128 x 256 (8 waves), chunks of one, a few and many passes, ragged last
+rows and the three forms of dL/dout, against float64 products of the same
+tensors and stash (/root/reference/mlp_fused.md:88-95).  Tolerances: 16-bit as in
+test_wide_gpu.py (2e-2 |ref| + 2e-3 max|ref|, Frobenius 1e-2; bf16 three
+times that), fp32 as in test_fp32_gpu.py (1e-3, 1e-4, 5e-4)."""
+import numpy as np
+import pytest
+import torch
+
+from mlpmk import ops
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # fp32: QUAD below 32,768 rows, PAIR from there (not below 64 features)
+    ((128, 128, 128, 128), 32767, "f32"), ((128, 128, 128, 128), 32768, "f32"), ((128, 128, 128, 128), 65600, "f32"),
+    ((32, 80, 112, 96, 24), 40001, "f32"), ((64, 64, 48, 8), 40001, "f32"), ((128, 128, 16), 70001, "f32"),
+    # widths above 128: QUAD below 24,576, WIDE from there
+    ((128, 256, 256, 128), 24575, "f16"), ((128, 256, 256, 128), 24576, "f16"), ((128, 256, 256, 128), 24701, "bf16"),
+    ((144, 208, 16, 256, 136), 30001, "f16"), ((256, 256, 8), 25000, "bf16"), ((16, 144, 144, 144, 144, 72), 26000, "f16"),
+    # data-gradient tiles: 32 rows up to 16,384, 64 from there
+    ((128, 256, 256, 128), 16384, "f16"), ((128, 256, 256, 128), 16385, "f16"), ((96, 160, 104), 3, "f16"),
+    ((128, 128, 128, 128), 33, "f16"), ((64, 128, 64, 32, 128, 120), 16449, "f32"),
+]
+
+
+@pytest.mark.parametrize("dims,m,elem", CASES)
+@pytest.mark.parametrize("how", ["dense", "row", "scalar"])
+def test_two_pass_backward_forms(dims, m, elem, how):
+    dt = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}[elem]
+    rng = np.random.default_rng(m)
+    x = torch.from_numpy(rng.standard_normal((m, dims[0]), dtype=np.float32)).to(dt)
+    ws = [torch.from_numpy(rng.standard_normal((dims[i], dims[i + 1]), dtype=np.float32) / np.sqrt(dims[i])).to(dt)
+          for i in range(len(dims) - 1)]
+    xd, wd = x.cuda(), [w.cuda() for w in ws]
+    _, hs = ops.fwd(xd, wd, stash=True)
+    shape = {"dense": (m, dims[-1]), "row": (1, dims[-1]), "scalar": (1, 1)}[how]
+    dout = torch.from_numpy(rng.standard_normal(shape, dtype=np.float32)).to(dt).cuda().expand(m, dims[-1])
+    dws = [torch.full(tuple(w.shape), float("nan"), device="cuda") for w in ws]
+    dx = torch.empty_like(xd)
+    ops.bwd(xd, wd, hs, dout, dws, dx, accumulate=False)
+    # float64 gradients of the same stash, on the GPU (plain products)
+    dz = dout.double()
+    tol, scale_tol, fro = {"f16": (2e-2, 2e-3, 1e-2), "bf16": (6e-2, 6e-3, 3e-2), "f32": (1e-3, 1e-4, 5e-4)}[elem]
+    for l in range(len(ws) - 1, -1, -1):
+        a = hs[l - 1].double() if l > 0 else xd.double()
+        ref = a.t().contiguous() @ dz.contiguous()
+        err = (dws[l].double() - ref).abs()
+        assert bool((err <= tol * ref.abs() + scale_tol * ref.abs().max()).all()), f"dW{l + 1}: {err.max().item()}"
+        assert (err.norm() / ref.norm()).item() <= fro, f"dW{l + 1}"
+        dh = dz @ wd[l].double().t().contiguous()
+        dz = dh * -torch.expm1(-hs[l - 1].double()) if l > 0 else dh
+    rows = dz.abs().amax(dim=1, keepdim=True)
+    assert bool(((dx.double() - dz).abs() <= max(tol / 2, 2e-4) * (dz.abs() + rows)).all()), "dx"
