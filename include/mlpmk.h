@@ -357,6 +357,20 @@ int mlpmk_sigmoid_h_mul(const float* h, const void* dh, int dh_dtype, float* dz3
 int mlpmk_softplus_f32(const float* z, float* h, int64_t n, void* stream);
 
 /*
+ * Element conversions of up to 16 matrices in one launch: dst[i] (16-byte
+ * aligned, contiguous, dst_rows x dst_cols of dst_dtype[i]) takes src[i]
+ * (contiguous, src_rows x src_cols of src_dtype[i]) rounded to nearest even,
+ * cropped to dst's size, zeros past src's.  shapes holds src_rows, src_cols,
+ * dst_rows, dst_cols of each.  The casts and paddings around the other entry
+ * points (the reference leaves its INPUT_DTYPE casts to the framework, a
+ * launch per tensor: /root/reference/mlp_fused.md:159-172).
+ * MLPMK_ERR_UNSUPPORTED_SHAPE for tensors of 2^31 elements or more.  Since
+ * ABI version 205.
+ */
+int mlpmk_convert(int n, const void* const* src, const int* src_dtype, void* const* dst, const int* dst_dtype,
+                  const int64_t* shapes, void* stream);
+
+/*
  * Diagnostic: a streaming copy of `bytes` bytes (multiple of 16) with the same
  * 128-bit load/store width and cache policy as the forward megakernel's x and
  * out traffic (default loads, non-temporal stores).  Used to calibrate

@@ -138,7 +138,10 @@ def _fused_mlp_fwd(x, w1, w2, w3):
     if route > 0:
         # Input width not a multiple of 16: zero columns of x and zero rows of
         # W1 add nothing to x @ W1.
-        x, w1 = F.pad(x, (0, route)), F.pad(w1, (0, 0, 0, route))
+        if w1.dtype == x.dtype:
+            x, (w1,) = _ops.as_inputs(x, [w1], x.dtype, route)
+        else:  # (rejected by fwd_into, with its own message)
+            x, w1 = F.pad(x, (0, route)), F.pad(w1, (0, 0, 0, route))
     elif route < 0:
         from mlpmk import fallback
 

@@ -56,6 +56,7 @@ SIGNATURES = {
     ),
     "mlpmk_copy": (c_int, [c_void_p, c_void_p, c_int64, c_void_p]),
     "mlpmk_sigmoid_h_mul": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int64, c_void_p]),
+    "mlpmk_convert": (c_int, [c_int, P_VOIDP, P_INT, P_VOIDP, P_INT, ctypes.POINTER(c_int64), c_void_p]),
     "mlpmk_softplus_f32": (c_int, [c_void_p, c_void_p, c_int64, c_void_p]),
 }
 

@@ -41,7 +41,6 @@ library's elementwise kernels.
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 from torch.autograd.function import once_differentiable
 
 from . import _lib, ops
@@ -161,11 +160,6 @@ def _input_pad(dims, dtype):
     return 0 if _layerwise((d0 + pad,) + tuple(dims[1:]), dtype) else pad
 
 
-def _padded(x, w0, pad):
-    """``x`` with ``pad`` zero columns and ``w0`` with ``pad`` zero rows."""
-    return F.pad(x, (0, pad)), F.pad(w0, (0, 0, 0, pad))
-
-
 def _needs_graph(*tensors):
     """True when autograd will run a backward through this call."""
     return torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
@@ -198,13 +192,10 @@ class FusedMLPFunction(torch.autograd.Function):
     def forward(ctx, x, *weights):
         dims = (int(x.shape[1]),) + tuple(int(w.shape[1]) for w in weights)
         dt = kernel_dtype(x, dims)
-        x = x.to(dt).contiguous()
-        weights = [w.to(dt).contiguous() for w in weights]
         pad = _input_pad(dims, dt)
-        if pad:
-            x, w0 = _padded(x, weights[0], pad)
-            weights = [w0] + weights[1:]
-            dims = (dims[0] + pad,) + dims[1:]
+        ctx.w_dtypes = [w.dtype for w in weights]
+        x, weights = ops.as_inputs(x, list(weights), dt, pad)
+        dims = (dims[0] + pad,) + dims[1:]
         if any(ctx.needs_input_grad):
             rc = _use_recompute(dims, int(x.shape[0]), ctx.needs_input_grad[0], dt)
             if _layerwise(dims, dt):
@@ -254,7 +245,17 @@ class FusedMLPFunction(torch.autograd.Function):
             d0 = dims[0] - ctx.pad
             dx = dx[:, :d0] if dx is not None else None
             dws[0] = dws[0][:d0]
-        return (dx, *[d if need else None for d, need in zip(dws, ctx.needs_input_grad[1:])])
+        # The gradients in their weights' own types, in one launch (autograd
+        # would convert them one by one).
+        grads, todo = [], []
+        for d, dt, need in zip(dws, ctx.w_dtypes, ctx.needs_input_grad[1:]):
+            if need and dt in (torch.float16, torch.bfloat16):
+                g = torch.empty(d.shape, dtype=dt, device=d.device)
+                todo.append((d, g))
+                d = g
+            grads.append(d if need else None)
+        ops.convert(todo, x.device)
+        return (dx, *grads)
 
 
 class FusedMLPWNFunction(torch.autograd.Function):
@@ -299,9 +300,7 @@ class FusedMLPWNFunction(torch.autograd.Function):
         if pad:
             # Input width padded to a multiple of 16 (zero columns of x, zero
             # rows of W_1) so that the fused kernels take the network.
-            ws = _split(w_all, dims)
-            xp, w0 = _padded(x, ws[0], pad)
-            ws = [w0] + ws[1:]
+            xp, ws = ops.as_inputs(x, _split(w_all, dims), x.dtype, pad)
             if any(ctx.needs_input_grad):
                 pdims = (dims[0] + pad,) + dims[1:]
                 rc = _use_recompute(pdims, M, ctx.needs_input_grad[0], x.dtype)
@@ -354,7 +353,9 @@ class FusedMLPWNFunction(torch.autograd.Function):
             # and its first rows copied into the flat block, dx cut back.
             pdims = (dims[0] + ctx.pad,) + dims[1:]
             ws = _split(w_all, dims)
-            ws = [F.pad(ws[0], (0, 0, 0, ctx.pad))] + ws[1:]
+            w0 = torch.empty((pdims[0], dims[1]), dtype=x.dtype, device=dev)
+            ops.convert([(ws[0], w0)], dev)
+            ws = [w0] + ws[1:]
             dw_all = torch.empty(nw, dtype=torch.float32, device=dev)
             dws = _split(dw_all, dims)
             dw0 = torch.empty((pdims[0], dims[1]), dtype=torch.float32, device=dev)
@@ -423,12 +424,10 @@ def fused_mlp(x, *weights):
         return FusedMLPFunction.apply(x, *weights)
     dims = (int(x.shape[1]),) + tuple(int(w.shape[1]) for w in weights)
     dt = kernel_dtype(x, dims)
-    x = x.to(dt).contiguous()
-    weights = [w.to(dt).contiguous() for w in weights]
     pad = _input_pad(dims, dt)
+    x, weights = ops.as_inputs(x, list(weights), dt, pad)
     if pad:
-        x, w0 = _padded(x, weights[0], pad)
-        return ops.fwd(x, [w0] + weights[1:])
+        return ops.fwd(x, weights)
     if _layerwise(dims, dt):
         from . import fallback
 
@@ -448,9 +447,7 @@ def fused_mlp_wn(x, v_all, g_all, dims):
     ops.wn_fwd(dims, v_all.contiguous(), g_all.contiguous(), w_all, inv_all)
     pad = _input_pad(dims, x.dtype)
     if pad:
-        ws = _split(w_all, dims)
-        xp, w0 = _padded(x, ws[0], pad)
-        return ops.fwd(xp, [w0] + ws[1:])
+        return ops.fwd(*ops.as_inputs(x, _split(w_all, dims), x.dtype, pad))
     if _layerwise(dims, x.dtype):
         from . import fallback
 

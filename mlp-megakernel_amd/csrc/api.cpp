@@ -30,6 +30,8 @@ int wn_fwd_dispatch(int L, const int* dims, int dtype, int w_dtype, const void* 
 int wn_bwd_dispatch(int L, const int* dims, int dtype, const float* dw, const void* v, const void* g,
                     const float* inv_norm, void* dv, void* dg, hipStream_t st);
 int copy_dispatch(const void* src, void* dst, int64_t bytes, hipStream_t st);
+int convert_dispatch(int n, const void* const* src, const int* src_dt, void* const* dst, const int* dst_dt,
+                     const int64_t* shapes, hipStream_t st);
 int softplus_f32_dispatch(const float* z, float* h, int64_t n, hipStream_t st);
 int sigmoid_h_mul_dispatch(const float* h, const void* dh, int dh_dtype, float* dz32, void* dz16, int dz16_dtype,
                            int64_t n, hipStream_t st);
@@ -119,7 +121,7 @@ using namespace mlpmk;
 
 extern "C" {
 
-int mlpmk_version(void) { return 205; }  // 2.05: mlpmk_fwd_layers (2.04: mlpmk_softplus_f32, mlpmk_fwd_supported_dtype 2.03: MLPMK_BWD_WRITE_DW)
+int mlpmk_version(void) { return 205; }  // 2.05: mlpmk_fwd_layers, mlpmk_convert (2.04: mlpmk_softplus_f32, mlpmk_fwd_supported_dtype 2.03: MLPMK_BWD_WRITE_DW)
 
 const char* mlpmk_status_string(int status) {
   switch (status) {
@@ -441,6 +443,29 @@ int mlpmk_softplus_f32(const float* z, float* h, int64_t n, void* stream) {
   int rc;
   if ((rc = check_ptr(z, "z")) || (rc = check_ptr(h, "h"))) return rc;
   return softplus_f32_dispatch(z, h, n, static_cast<hipStream_t>(stream));
+}
+
+int mlpmk_convert(int n, const void* const* src, const int* src_dtype, void* const* dst, const int* dst_dtype,
+                  const int64_t* shapes, void* stream) {
+  g_last_error[0] = 0;
+  if (n < 0 || n > 16) return fail(MLPMK_ERR_INVALID_ARG, "n=%d (0..16 tensors)", n);
+  if (n > 0 && (!src || !src_dtype || !dst || !dst_dtype || !shapes))
+    return fail(MLPMK_ERR_INVALID_ARG, "a NULL argument array");
+  for (int i = 0; i < n; ++i) {
+    int rc;
+    if ((rc = check_fwd_dtype(src_dtype[i])) || (rc = check_fwd_dtype(dst_dtype[i]))) return rc;
+    for (int k = 0; k < 4; ++k)
+      if (shapes[4 * i + k] < 0)
+        return fail(MLPMK_ERR_INVALID_ARG, "shapes[%d]=%lld is negative", 4 * i + k, (long long)shapes[4 * i + k]);
+    if (shapes[4 * i + 2] == 0 || shapes[4 * i + 3] == 0) continue;
+    if ((rc = check_ptr(dst[i], "dst"))) return rc;
+    const uintptr_t al = src_dtype[i] == MLPMK_DTYPE_F32 ? 3u : 1u;
+    if (!src[i] && shapes[4 * i] > 0 && shapes[4 * i + 1] > 0) return fail(MLPMK_ERR_INVALID_ARG, "src is NULL");
+    if (reinterpret_cast<uintptr_t>(src[i]) & al)
+      return fail(MLPMK_ERR_MISALIGNED, "src=%p is not aligned to its elements", src[i]);
+  }
+  if (n == 0) return MLPMK_OK;
+  return convert_dispatch(n, src, src_dtype, dst, dst_dtype, shapes, static_cast<hipStream_t>(stream));
 }
 
 int mlpmk_copy(const void* src, void* dst, int64_t bytes, void* stream) {

@@ -227,6 +227,62 @@ def _wn_bwd_raw(dev, dims, pcode, dw_ptr, v_ptr, g_ptr, inv_ptr, dv_ptr, dg_ptr)
         _check("mlpmk_wn_bwd", rc)
 
 
+_CODES = {torch.float32: _lib.DTYPE_F32, torch.float16: _lib.DTYPE_F16, torch.bfloat16: _lib.DTYPE_BF16}
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _convertible(src, dev):
+    return (type(src) in _PLAIN and src.dim() == 2 and src.dtype in _CODES and src.device == dev
+            and src.is_contiguous() and src.numel() < 1 << 31)
+
+
+def convert(pairs, dev):
+    """``dst`` takes ``src`` (matrices) converted to its type, cropped to its
+    shape and zero past src's, for every ``(src, dst)`` of ``pairs``: one
+    launch (``mlpmk_convert``) where every pair is contiguous, on ``dev`` and
+    of a type the library knows, else torch operations.  The destinations are
+    fresh contiguous tensors of the caller."""
+    if not pairs:
+        return
+    if len(pairs) <= 16 and dev.type == "cuda" and all(
+            _convertible(s, dev) and d.dtype in _CODES and d.numel() < 1 << 31 for s, d in pairs):
+        n = len(pairs)
+        shapes = [v for s, d in pairs for v in (s.shape[0], s.shape[1], d.shape[0], d.shape[1])]
+        rc = _launch(dev, _lib.get().mlpmk_convert, n, (_lib.c_void_p * n)(*[s.data_ptr() for s, _ in pairs]),
+                     (_lib.c_int * n)(*[_CODES[s.dtype] for s, _ in pairs]),
+                     (_lib.c_void_p * n)(*[d.data_ptr() for _, d in pairs]),
+                     (_lib.c_int * n)(*[_CODES[d.dtype] for _, d in pairs]), (_lib.c_int64 * (4 * n))(*shapes))
+        if rc:
+            _check("mlpmk_convert", rc)
+        return
+    for s, d in pairs:
+        r, c = min(s.shape[0], d.shape[0]), min(s.shape[1], d.shape[1])
+        if (r, c) != tuple(d.shape):
+            d.zero_()
+        d[:r, :c].copy_(s[:r, :c])
+
+
+def as_inputs(x, weights, dt, pad=0):
+    """``x`` and the weights as contiguous ``dt`` tensors, ``x`` with ``pad``
+    zero columns and the first weight with ``pad`` zero rows appended; what is
+    already so is returned as it is, the rest goes through one ``convert``."""
+    todo, res = [], []
+    for i, t in enumerate([x] + weights):
+        p = pad if i < 2 else 0
+        if t.dtype == dt and not p:
+            res.append(t.contiguous())
+            continue
+        if t.dim() != 2:  # (the callers' own checks name it)
+            res.append(t.to(dt).contiguous())
+            continue
+        rows, cols = int(t.shape[0]), int(t.shape[1])
+        d = torch.empty((rows, cols + p) if i == 0 else (rows + p, cols), dtype=dt, device=t.device)
+        todo.append((t.contiguous(), d))
+        res.append(d)
+    convert(todo, x.device)
+    return res[0], res[1:]
+
+
 DOUT_SCALAR = -1  # MLPMK_DOUT_SCALAR
 
 
@@ -250,8 +306,8 @@ def _dout_rows(dout, M, out_w, dtype, dev):
         # The library reads dout rows from 16-byte boundaries: an output width
         # that is not a multiple of 8, or rows that start off such a boundary,
         # get a padded copy.
-        padded = torch.zeros((M, -(-out_w // 8) * 8), dtype=dtype, device=dev)
-        padded[:, :out_w] = dout
+        padded = torch.empty((M, -(-out_w // 8) * 8), dtype=dtype, device=dev)
+        convert([(dout, padded)], dev)
         dout, row_stride = padded, padded.shape[1]
     return dout, row_stride
 
