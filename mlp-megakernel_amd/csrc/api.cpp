@@ -24,6 +24,7 @@ bool bwd_recompute_supported(int L, const int* dims);
 int bwd_dispatch(int L, const int* dims, const BwdParams& p, int dtype, hipStream_t st);
 int bwd_clear_dw(int L, const int* dims, float* const* dw, hipStream_t st);
 int bwd_workspace_bytes(int L, const int* dims, int64_t M, bool dx, int dtype, int64_t* bytes);
+int64_t bwd_workspace_optional(int L, const int* dims, int64_t M, int dtype);
 int scratch_workspace(void** ptr, int64_t* bytes);
 int wn_fwd_dispatch(int L, const int* dims, int dtype, int w_dtype, const void* v, const void* g, void* w_out,
                     float* inv_norm, hipStream_t st);
@@ -335,6 +336,8 @@ static int bwd_common(int num_layers, const int* dims, int dtype, const void* x,
     if ((rc = check_ptr(workspace, "workspace"))) return rc;
     int64_t need = 0;
     if ((rc = bwd_workspace_bytes(num_layers, dims, M, dx != nullptr, dtype, &need))) return rc;
+    p.pack_room = workspace_bytes >= need;
+    need -= bwd_workspace_optional(num_layers, dims, M, dtype);
     if (use_scratch && need > workspace_bytes)
       return fail(MLPMK_ERR_UNSUPPORTED_SHAPE,
                   "M=%lld needs %lld bytes of workspace; mlpmk_bwd_noalloc's scratch holds %lld "

@@ -1455,6 +1455,7 @@ static int bwd_workspace_t(int L, const int* dims, int64_t M, bool dx, int64_t* 
 
 bool tp_supported(int L, const int* dims, int dtype);
 int tp_workspace_bytes(int L, const int* dims, int dtype, int64_t M, int64_t* bytes);
+int64_t tp_pack_bytes(int L, const int* dims, int dtype, int64_t M);
 int tp_dispatch(int L, const int* dims, int dtype, const BwdParams& bp, void* ws, hipStream_t st);
 
 static bool fused_supported(int L, const int* dims) {
@@ -1495,6 +1496,13 @@ int bwd_workspace_bytes(int L, const int* dims, int64_t M, bool dx, int dtype, i
   }
   *bytes = fused > two ? fused : two;
   return MLPMK_OK;
+}
+
+// How much of bwd_workspace_bytes a call can do without (the packed weights of
+// the two-pass backward, the last part of its workspace).
+int64_t bwd_workspace_optional(int L, const int* dims, int64_t M, int dtype) {
+  const bool fused = dtype != MLPMK_DTYPE_F32 && fused_supported(L, dims);
+  return !fused && bwd_path(L, dims, dtype, M, false) == 1 ? tp_pack_bytes(L, dims, dtype, M) : 0;
 }
 
 // Library-owned workspace of mlpmk_bwd_noalloc, for callers that cannot

@@ -100,6 +100,32 @@ struct DgGeo {
   }
 };
 
+// Packed weights of a layer (16-bit tensors): fragment (mb, s), 1 KiB, holds in
+// lane (i, g) W_l[outfeat(mb, i)][16s + 8g + 0..7]; K-steps padded with zeros
+// to whole turns of 4.
+__host__ __device__ constexpr int pack_ks(int nout) { return (nout + 63) / 64 * 4; }
+__host__ __device__ constexpr int pack_frags(int k, int nout) { return (k + 31) / 32 * pack_ks(nout); }
+struct PackParams {
+  const f16* w[kMaxLayersHost];
+  f16* dst[kMaxLayersHost];
+  int first[kMaxLayersHost + 1];  // first fragment lane of layer l
+  int dims[kMaxLayersHost + 1];
+  int L;
+};
+__global__ __launch_bounds__(256) void tp_pack_kernel(PackParams p) {
+  const int t = blockIdx.x * 256 + threadIdx.x;
+  if (t >= p.first[p.L]) return;
+  int l = 0;
+  while (l + 1 < p.L && t >= p.first[l + 1]) ++l;
+  const int K = p.dims[l], Nout = p.dims[l + 1], KP = pack_ks(Nout);
+  const int item = t - p.first[l], f = item >> 6, lane = item & 63;
+  const int row = outfeat(f / KP, lane & 31), c = 16 * (f % KP) + 8 * (lane >> 5);
+  // (widths here are multiples of 8: a piece lies in the row or past it)
+  f16x8 v = {};
+  if (row < K && c < Nout) v = *reinterpret_cast<const f16x8*>(p.w[l] + (int64_t)row * Nout + c);
+  *reinterpret_cast<f16x8*>(p.dst[l] + (int64_t)item * 8) = v;
+}
+
 // A workgroup of NWV waves runs tiles of 32 RB rows, one after the other; wave w
 // owns features [32w, 32w + 32) of every data gradient and all rows of the
 // tile.  dL/dout and every dz_l go through LDS tiles (two, in turns: one
@@ -112,8 +138,12 @@ struct DgGeo {
 // RES: every layer's fragments stay in registers for the whole kernel
 // (loaded once per workgroup); otherwise they are read from L2 through a ring
 // of kRing K-steps, the next layer's first ones requested before this layer's
-// results are evaluated.
-template <class N, int EM, bool DX, bool RES, int RB>
+// results are evaluated.  PK: from the packed copy (tp_pack_kernel), 1 KiB
+// whole; from W_l itself a fragment is 32 bytes of each of 32 rows, and at
+// width 256 the 8 waves' rows do not stay in the vector cache until the
+// K-steps that use the rest of their lines (128-256-256-128 bf16 at 100,003
+// rows: this pass 101 -> 80 us, the packing 4.7).
+template <class N, int EM, bool DX, bool RES, int RB, bool PK>
 struct DgWave {
   using G = DgGeo<N, DX>;
   static constexpr int L = N::L, CH = G::CH, NT = EM == EM_F32 ? 2 : 1;
@@ -158,6 +188,11 @@ struct DgWave {
   template <int l>
   __device__ __forceinline__ Raw load_frag(int s) const {
     const int K = dimw<N>(p, l), Nout = dimw<N>(p, l + 1);
+    if constexpr (PK) {  // (a wave past the layer's width, a K-step past the padded width: past the resource)
+      const int KP = pack_ks(Nout);
+      const rsrc_t r = make_rsrc(p.wp[l], (uint32_t)(pack_frags(K, Nout) * 1024));
+      return load_raw(r, s < KP ? (uint32_t)((w * KP + s) * 64 + lane) * 16u : kPast);
+    }
     const rsrc_t r = make_rsrc(p.w[l], (uint32_t)(K * Nout * kEs<EM>));
     const int c = 16 * s + 8 * g;
     const uint32_t off = (uint32_t)(outfeat(w, n) * Nout + c) * kEs<EM>;
@@ -359,10 +394,10 @@ struct DgWave {
   }
 };
 
-template <class N, int EM, bool DX, bool RES, int RB>
+template <class N, int EM, bool DX, bool RES, int RB, bool PK>
 __global__ __launch_bounds__((DgGeo<N, DX>::NWV * 64)) void tp_dgrad_kernel(TpParams p) {
   using G = DgGeo<N, DX>;
-  using W = DgWave<N, EM, DX, RES, RB>;
+  using W = DgWave<N, EM, DX, RES, RB, PK>;
   static_assert(G::valid(), "two-pass backward shape");
   __shared__ f16x8 tile[2][W::NT][W::ROWS * G::CH];  // two exchange tiles (hi, and lo with fp32 tensors)
   const int lane = threadIdx.x & 63;
@@ -736,10 +771,10 @@ int cached_occupancy(const void* kern, int threads, int* occ_out) {
   return MLPMK_OK;
 }
 
-template <class N, int EM, bool DX, bool RES, int RB>
+template <class N, int EM, bool DX, bool RES, int RB, bool PK = false>
 int launch_dgrad_rb(const TpParams& p, int cus, hipStream_t st) {
   using G = tp::DgGeo<N, DX>;
-  const void* kern = reinterpret_cast<const void*>(&tp::tp_dgrad_kernel<N, EM, DX, RES, RB>);
+  const void* kern = reinterpret_cast<const void*>(&tp::tp_dgrad_kernel<N, EM, DX, RES, RB, PK>);
   int occ = 0;
   int rc = cached_occupancy(kern, G::NWV * 64, &occ);
   if (rc != MLPMK_OK) return rc;
@@ -747,7 +782,7 @@ int launch_dgrad_rb(const TpParams& p, int cus, hipStream_t st) {
   const int64_t cap = (int64_t)cus * occ;
   const int grid = (int)(ntiles < cap ? ntiles : cap);
   (void)hipGetLastError();
-  hipLaunchKernelGGL((tp::tp_dgrad_kernel<N, EM, DX, RES, RB>), dim3(grid), dim3(G::NWV * 64), 0, st, p);
+  hipLaunchKernelGGL((tp::tp_dgrad_kernel<N, EM, DX, RES, RB, PK>), dim3(grid), dim3(G::NWV * 64), 0, st, p);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? MLPMK_OK : hip_fail(e, "two-pass dgrad kernel launch");
 }
@@ -755,6 +790,9 @@ int launch_dgrad_rb(const TpParams& p, int cus, hipStream_t st) {
 // Tiles of 64 rows where that still gives every CU one, else of 32 rows.
 template <class N, int EM, bool DX, bool RES>
 int launch_dgrad(const TpParams& p, int cus, hipStream_t st) {
+  if constexpr (EM != tp::EM_F32 && !RES) {
+    if (p.wp[0]) return launch_dgrad_rb<N, EM, DX, RES, 2, true>(p, cus, st);
+  }
   return p.M > (int64_t)64 * cus ? launch_dgrad_rb<N, EM, DX, RES, 2>(p, cus, st)
                                  : launch_dgrad_rb<N, EM, DX, RES, 1>(p, cus, st);
 }
@@ -907,11 +945,26 @@ bool tp_supported(int L, const int* dims, int dtype) {
   return dims[L] >= 8 && dims[L] <= wmax && dims[L] % 8 == 0;
 }
 
+// The packed weights' bytes, 0 where the pass takes them from W_l: fp32 tensors
+// (split when loaded), widths up to 128, and batches up to this many rows,
+// where the packing launch (4 us) costs more than it saves.
+constexpr int64_t kPackMinRows = 32768;
+int64_t tp_pack_bytes(int L, const int* dims, int dtype, int64_t M) {
+  int wmax = 0;
+  int64_t b = 0;
+  for (int l = 0; l < L; ++l) {
+    b += (int64_t)tp::pack_frags(dims[l], dims[l + 1]) * 1024;
+    wmax = dims[l] > wmax ? dims[l] : wmax;
+  }
+  wmax = dims[L] > wmax ? dims[L] : wmax;
+  return dtype != MLPMK_DTYPE_F32 && wmax > 128 && M >= kPackMinRows ? b : 0;
+}
+
 // Workspace of the two-pass backward: dz_0 .. dz_{L-2} ([M, d[l+1]] each,
-// 16-bit or fp32 elements, 256-byte aligned).
+// 16-bit or fp32 elements, 256-byte aligned), then the packed weights.
 int tp_workspace_bytes(int L, const int* dims, int dtype, int64_t M, int64_t* bytes) {
   const int es = dtype == MLPMK_DTYPE_F32 ? 4 : 2;
-  int64_t b = 0;
+  int64_t b = tp_pack_bytes(L, dims, dtype, M);
   for (int l = 0; l + 1 < L; ++l) b += round256(M * dims[l + 1] * es);
   *bytes = b;
   return MLPMK_OK;
@@ -941,6 +994,22 @@ int tp_dispatch(int L, const int* dims, int dtype, const BwdParams& bp, void* ws
   for (int l = 0; l + 1 < L; ++l) {
     p.dz[l] = c;
     c += round256(bp.M * dims[l + 1] * es);
+  }
+  if (bp.pack_room && tp_pack_bytes(L, dims, dtype, bp.M) > 0) {
+    tp::PackParams pk = {};
+    pk.L = L;
+    for (int l = 0; l < L; ++l) {
+      pk.w[l] = bp.w[l];
+      p.wp[l] = pk.dst[l] = reinterpret_cast<f16*>(c);
+      const int frags = tp::pack_frags(dims[l], dims[l + 1]);
+      pk.first[l + 1] = pk.first[l] + frags * 64;
+      c += (int64_t)frags * 1024;
+    }
+    for (int l = 0; l <= L; ++l) pk.dims[l] = dims[l];
+    (void)hipGetLastError();
+    hipLaunchKernelGGL(tp::tp_pack_kernel, dim3((pk.first[L] + 255) / 256), dim3(256), 0, st, pk);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return hip_fail(e, "weight packing kernel launch");
   }
   const int S = wgrad_chunks(L, dims, bp.M, dtype == MLPMK_DTYPE_F32, cus);
   const int em = dtype == MLPMK_DTYPE_F32 ? tp::EM_F32 : dtype == MLPMK_DTYPE_BF16 ? tp::EM_BF16 : tp::EM_F16;

@@ -37,6 +37,9 @@ struct BwdParams {
   // blocks back to back, at part + b * (sum_l d[l] * d[l+1]), and a second
   // kernel sums the partials into dw.
   float* part;
+  // Two-pass backward: the workspace has room for the packed weights as well
+  // (bwd_workspace_optional bytes at its end).
+  int pack_room;
   // Segment mode only (the upper layers of a deeper network): the fp32
   // activation feeding layer 0, h_{l0} of the full network, in place of x.
   const float* h0;
@@ -61,6 +64,7 @@ struct TpParams {
   void* dx;                            // nullable
   float* dw[kMaxLayersHost];           // fp32 [d[l], d[l+1]], accumulated into (fp32 atomics)
   void* dz[kMaxLayersHost];            // dz_l, l = 0 .. L-2: [M, d[l+1]] in the workspace
+  const void* wp[kMaxLayersHost];      // W_l in data-gradient operand order (tp_pack_kernel), in the workspace
   int64_t M;
   // Nonzero: the data-gradient pass clears dw before the weight-gradient
   // pass adds to it (MLPMK_BWD_WRITE_DW).
