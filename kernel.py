@@ -126,7 +126,7 @@ def _fused_mlp_fwd(x, w1, w2, w3):
     """Inference forward: one kernel launch, no intermediate in global memory
     (an input width that is not a multiple of 16 is zero-padded to one first;
     networks no fused kernel takes -- fp32 ones wider than 128, any wider
-    than 256 -- run layer by layer: mlpmk.fallback.fwd)."""
+    than 256 -- run through mlpmk.fallback.fwd)."""
     x = x.contiguous()
     w1, w2, w3 = w1.contiguous(), w2.contiguous(), w3.contiguous()
     M = x.shape[0]

@@ -22,10 +22,11 @@ Training path of the reference's ``FusedMLPSoftplus`` / ``FusedMLPSoftplusWN``
   INPUT_DTYPE kernels do (mlp_fused.md:159-166): fp32 parameters and an fp32
   ``x`` run the fp32-tensor kernels (bf16 hi/lo split operands: fp32's
   exponent range) and return an fp32 ``out``.  Networks no fused forward
-  takes (fp32 ones wider than 128, any wider than 256) run layer by layer
-  (``fallback.fwd``: fp32 library GEMMs, the library's fp32 softplus kernel,
-  hidden values rounded to the tensor format between layers) and train
-  through the fallback backward.
+  takes (fp32 ones wider than 128, any wider than 256) run through
+  ``fallback.fwd`` (16-bit ones up to 512 wide in one launch, else fp32
+  library GEMMs and the library's fp32 softplus kernel; hidden values rounded
+  to the tensor format between layers) and train through the fallback
+  backward.
 * inference: ``fused_mlp`` / ``fused_mlp_wn`` (and the modules) call the plain
   forward, without the fp32 stash, whenever autograd will not need it -- grad
   disabled (``torch.no_grad`` / ``inference_mode``) or nothing requiring grad.
@@ -138,8 +139,7 @@ _fwd_shapes = {}
 def _layerwise(dims, dtype):
     """True when no fused forward takes ``dims`` for ``dtype`` tensors (fp32
     networks wider than 128, any network wider than 256 or deeper than the
-    kernels' 5 layers): they run layer by layer (``fallback.fwd``: fp32
-    library GEMMs and the library's fp32 softplus kernel)."""
+    kernels' 5 layers): they run through ``fallback.fwd``."""
     key = (tuple(dims), dtype)
     ok = _fwd_shapes.get(key)
     if ok is None:

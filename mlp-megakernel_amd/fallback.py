@@ -26,7 +26,8 @@ a comparator.  Same arguments and results as ``ops.bwd``.
 
 For networks no fused forward takes (fp32 tensors wider than 128, any
 tensors wider than 256 or deeper than 5 layers), :func:`fwd` is the matching
-forward: fp32 library GEMMs and this library's fp32 softplus kernel
+forward: one launch for 16-bit networks up to 512 wide (``mlpmk_fwd_layers``),
+else fp32 library GEMMs and this library's fp32 softplus kernel
 (``mlpmk_softplus_f32``); :func:`bwd` then runs the backward (every GEMM in
 fp32 for fp32 tensors).
 """
