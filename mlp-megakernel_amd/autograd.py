@@ -251,10 +251,12 @@ class FusedMLPFunction(torch.autograd.Function):
         for d, dt, need in zip(dws, ctx.w_dtypes, ctx.needs_input_grad[1:]):
             if need and dt in (torch.float16, torch.bfloat16):
                 g = torch.empty(d.shape, dtype=dt, device=d.device)
-                todo.append((d, g))
+                rows, cols = d.shape
+                todo += (d.data_ptr(), _lib.DTYPE_F32, g.data_ptr(), ops._CODES[dt], rows, cols, rows, cols)
                 d = g
             grads.append(d if need else None)
-        ops.convert(todo, x.device)
+        if todo:
+            ops._convert_raw(x.device, todo)
         return (dx, *grads)
 
 

@@ -25,12 +25,14 @@ typedef __typeof__(mlpmk_bwd) bwd_t;
 typedef __typeof__(mlpmk_bwd_ws) bwd_ws_t;
 typedef __typeof__(mlpmk_wn_fwd) wn_fwd_t;
 typedef __typeof__(mlpmk_wn_bwd) wn_bwd_t;
+typedef __typeof__(mlpmk_convert) convert_t;
 
 static fwd_t* g_fwd;
 static bwd_t* g_bwd;
 static bwd_ws_t* g_bwd_ws;
 static wn_fwd_t* g_wn_fwd;
 static wn_bwd_t* g_wn_bwd;
+static convert_t* g_convert;
 
 enum { kMaxDims = 16 };
 
@@ -96,9 +98,9 @@ static int check_bound(void* fn) {
 /* bind(fwd, bwd, bwd_ws, wn_fwd, wn_bwd): entry-point addresses. */
 static PyObject* py_bind(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
   (void)self;
-  if (check_nargs(nargs, 5, "bind")) return NULL;
-  void* a[5];
-  for (int i = 0; i < 5; ++i) {
+  if (check_nargs(nargs, 6, "bind")) return NULL;
+  void* a[6];
+  for (int i = 0; i < 6; ++i) {
     a[i] = PyLong_AsVoidPtr(args[i]);
     ERR_OUT();
     if (!a[i]) {
@@ -111,6 +113,7 @@ static PyObject* py_bind(PyObject* self, PyObject* const* args, Py_ssize_t nargs
   g_bwd_ws = (bwd_ws_t*)a[2];
   g_wn_fwd = (wn_fwd_t*)a[3];
   g_wn_bwd = (wn_bwd_t*)a[4];
+  g_convert = (convert_t*)a[5];
   Py_RETURN_NONE;
 }
 
@@ -225,12 +228,45 @@ static PyObject* py_wn_bwd(PyObject* self, PyObject* const* args, Py_ssize_t nar
   return PyLong_FromLong(rc);
 }
 
+/* convert(items, stream) -> status; items: a list of 8 ints per matrix: src,
+ * src_dtype, dst, dst_dtype, src_rows, src_cols, dst_rows, dst_cols */
+static PyObject* py_convert(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+  (void)self;
+  if (check_nargs(nargs, 2, "convert") || check_bound((void*)g_convert)) return NULL;
+  enum { kMax = 16 };
+  if (!PyList_Check(args[0]) || PyList_GET_SIZE(args[0]) % 8 != 0 || PyList_GET_SIZE(args[0]) > 8 * kMax) {
+    PyErr_SetString(PyExc_ValueError, "items must be a list of 8 ints for each of up to 16 matrices");
+    return NULL;
+  }
+  const int n = (int)(PyList_GET_SIZE(args[0]) / 8);
+  const void* src[kMax];
+  void* dst[kMax];
+  int sd[kMax], dd[kMax];
+  int64_t shapes[4 * kMax];
+  for (int i = 0; i < n; ++i) {
+    src[i] = PyLong_AsVoidPtr(PyList_GET_ITEM(args[0], 8 * i));
+    sd[i] = (int)PyLong_AsLong(PyList_GET_ITEM(args[0], 8 * i + 1));
+    dst[i] = PyLong_AsVoidPtr(PyList_GET_ITEM(args[0], 8 * i + 2));
+    dd[i] = (int)PyLong_AsLong(PyList_GET_ITEM(args[0], 8 * i + 3));
+    for (int k = 0; k < 4; ++k) shapes[4 * i + k] = PyLong_AsLongLong(PyList_GET_ITEM(args[0], 8 * i + 4 + k));
+    ERR_OUT();
+  }
+  void* stream = as_ptr(args[1]);
+  ERR_OUT();
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = g_convert(n, src, sd, dst, dd, shapes, stream);
+  Py_END_ALLOW_THREADS
+  return PyLong_FromLong(rc);
+}
+
 static PyMethodDef kMethods[] = {
-    {"bind", (PyCFunction)(void (*)(void))py_bind, METH_FASTCALL, "bind(fwd, bwd, bwd_ws, wn_fwd, wn_bwd)"},
+    {"bind", (PyCFunction)(void (*)(void))py_bind, METH_FASTCALL, "bind(fwd, bwd, bwd_ws, wn_fwd, wn_bwd, convert)"},
     {"fwd", (PyCFunction)(void (*)(void))py_fwd, METH_FASTCALL, "mlpmk_fwd"},
     {"bwd", (PyCFunction)(void (*)(void))py_bwd, METH_FASTCALL, "mlpmk_bwd / mlpmk_bwd_ws"},
     {"wn_fwd", (PyCFunction)(void (*)(void))py_wn_fwd, METH_FASTCALL, "mlpmk_wn_fwd"},
     {"wn_bwd", (PyCFunction)(void (*)(void))py_wn_bwd, METH_FASTCALL, "mlpmk_wn_bwd"},
+    {"convert", (PyCFunction)(void (*)(void))py_convert, METH_FASTCALL, "mlpmk_convert"},
     {NULL, NULL, 0, NULL}};
 
 static struct PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_mlpmk_launch", NULL, -1, kMethods,

@@ -159,7 +159,7 @@ def _fast():
     if _shim_lib is not lib:
         addr = lambda f: ctypes.cast(f, ctypes.c_void_p).value  # noqa: E731
         _shim.bind(addr(lib.mlpmk_fwd), addr(lib.mlpmk_bwd), addr(lib.mlpmk_bwd_ws), addr(lib.mlpmk_wn_fwd),
-                   addr(lib.mlpmk_wn_bwd))
+                   addr(lib.mlpmk_wn_bwd), addr(lib.mlpmk_convert))
         _shim_lib = lib
     return _shim
 
@@ -244,17 +244,16 @@ def convert(pairs, dev):
     fresh contiguous tensors of the caller."""
     if not pairs:
         return
-    if len(pairs) <= 16 and dev.type == "cuda" and all(
-            _convertible(s, dev) and d.dtype in _CODES and d.numel() < 1 << 31 for s, d in pairs):
-        n = len(pairs)
-        shapes = [v for s, d in pairs for v in (s.shape[0], s.shape[1], d.shape[0], d.shape[1])]
-        rc = _launch(dev, _lib.get().mlpmk_convert, n, (_lib.c_void_p * n)(*[s.data_ptr() for s, _ in pairs]),
-                     (_lib.c_int * n)(*[_CODES[s.dtype] for s, _ in pairs]),
-                     (_lib.c_void_p * n)(*[d.data_ptr() for _, d in pairs]),
-                     (_lib.c_int * n)(*[_CODES[d.dtype] for _, d in pairs]), (_lib.c_int64 * (4 * n))(*shapes))
-        if rc:
-            _check("mlpmk_convert", rc)
-        return
+    if len(pairs) <= 16 and dev.type == "cuda":
+        items = []
+        for s, d in pairs:
+            if not _convertible(s, dev) or d.dtype not in _CODES or d.numel() >= 1 << 31:
+                items = None
+                break
+            items += (s.data_ptr(), _CODES[s.dtype], d.data_ptr(), _CODES[d.dtype], *s.shape, *d.shape)
+        if items is not None:
+            _convert_raw(dev, items)
+            return
     for s, d in pairs:
         r, c = min(s.shape[0], d.shape[0]), min(s.shape[1], d.shape[1])
         if (r, c) != tuple(d.shape):
@@ -281,6 +280,23 @@ def as_inputs(x, weights, dt, pad=0):
         res.append(d)
     convert(todo, x.device)
     return res[0], res[1:]
+
+
+def _convert_raw(dev, items):
+    """``mlpmk_convert`` of ``items``: 8 ints per matrix (source pointer and
+    type, destination pointer and type, source rows and columns, destination
+    rows and columns)."""
+    f = _fast()
+    if f is not None:
+        rc = _launch(dev, f.convert, items)
+    else:
+        n = len(items) // 8
+        shapes = [v for i in range(n) for v in items[8 * i + 4 : 8 * i + 8]]
+        rc = _launch(dev, _lib.get().mlpmk_convert, n, (_lib.c_void_p * n)(*items[0::8]), (_lib.c_int * n)(*items[1::8]),
+                     (_lib.c_void_p * n)(*items[2::8]), (_lib.c_int * n)(*items[3::8]),
+                     (_lib.c_int64 * (4 * n))(*shapes))
+    if rc:
+        _check("mlpmk_convert", rc)
 
 
 DOUT_SCALAR = -1  # MLPMK_DOUT_SCALAR
