@@ -232,6 +232,17 @@ struct Wave {
             }
           }
       }
+      // Features that only pad the layer (softplus(0), or NaN where a row holds
+      // an infinity: inf * 0) are handed on as zeros, against zero weights.  A
+      // piece of 8 is a feature of the layer or past it as a whole.
+      if (active && 64 * f + 64 > N) {
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+          const bool past = 64 * f + 16 * a + 8 * g >= N;
+#pragma unroll
+          for (int b = 0; b < RBW; ++b) h16[b][a] = past ? f16x8{} : h16[b][a];
+        }
+      }
       __syncthreads();  // every wave has read the layer's inputs
       if (active) {
 #pragma unroll

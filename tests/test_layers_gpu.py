@@ -143,3 +143,41 @@ def test_calls_the_kernel_does_not_take_still_run():
     for got in (fallback.fwd(x, ws), fallback.fwd(x.clone(), ws), fallback.fwd(x3, ws).reshape(50, 64)):
         torch.testing.assert_close(got.double(), ref, atol=1e-2, rtol=1e-2)
     assert ops.fwd_supported([128, 512, 64]) is False
+
+
+def _classes(a):
+    """0 finite, 1 +inf, 2 -inf, 3 NaN"""
+    a = np.asarray(a, np.float32)
+    return np.where(np.isnan(a), 3, np.where(np.isposinf(a), 1, np.where(np.isneginf(a), 2, 0)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims", [(128, 272, 272, 128), (16, 264, 24, 8), (40, 288, 264, 8, 264, 5), (24, 320, 320, 16)])
+@pytest.mark.parametrize("elem", ["f16", "bf16"])
+def test_infinities_stay_where_the_oracle_has_them(dims, elem):
+    # Weights of one sign per output column, none of them zero: an infinite
+    # input (or a hidden value past the element type) gives +inf or softplus(-inf)
+    # = 0, and no inf - inf or inf * 0 on the way.  A feature that pads a hidden
+    # width must add nothing to that.
+    dt = torch.float16 if elem == "f16" else torch.bfloat16
+    m = 200
+    x, ws = orc.make_inputs(dims, m, seed=7, elem=elem)
+    rng = np.random.default_rng(8)
+    sign = [np.where(rng.random(d) < (0.25 if i else 0.0), -1.0, 1.0).astype(np.float32) for i, d in enumerate(dims[1:])]
+    ws = [orc.round_elem((np.abs(np.asarray(w, np.float32)) + 2.0 ** -6) * (0.125 if i else 1.0), elem) * s
+          for i, (w, s) in enumerate(zip(ws, sign))]
+    x = np.asarray(x, np.float32)
+    x[3, 5], x[70, 0], x[130, 2] = np.inf, -np.inf, np.nan
+    x[150] = orc.round_elem(np.abs(x[150]) * (3e4 if elem == "f16" else 1e38), elem)  # h past the largest element
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref, ref_h = orc.forward(x, ws, round_hidden=True, return_hidden=True, elem=elem)
+        ref = orc.round_elem(ref, elem)
+    assert (_classes(ref)[3] != 3).all() and (_classes(ref)[[3, 150]] == 1).any() and np.isfinite(ref[70]).all()
+    out, hs = fallback._fwd_layers(torch.from_numpy(x).cuda().to(dt), [torch.from_numpy(w).cuda().to(dt) for w in ws], True)
+    for got, want in zip([out, *hs], [ref, *ref_h]):
+        got = got.float().cpu().numpy()
+        assert np.array_equal(_classes(got), _classes(want))
+        fin = np.isfinite(want)
+        fin[150] = False
+        ok, err, _ = orc.allclose_report(got[fin], want[fin], 1e-2 if elem == "f16" else 3e-2, 1e-2 if elem == "f16" else 3e-2)
+        assert ok, err
