@@ -229,6 +229,7 @@ def _wn_bwd_raw(dev, dims, pcode, dw_ptr, v_ptr, g_ptr, inv_ptr, dv_ptr, dg_ptr)
 
 _CODES = {torch.float32: _lib.DTYPE_F32, torch.float16: _lib.DTYPE_F16, torch.bfloat16: _lib.DTYPE_BF16}
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
+_MAX_CONVERT = 16  # matrices of one mlpmk_convert call
 
 
 def _convertible(src, dev):
@@ -239,12 +240,12 @@ def _convertible(src, dev):
 def convert(pairs, dev):
     """``dst`` takes ``src`` (matrices) converted to its type, cropped to its
     shape and zero past src's, for every ``(src, dst)`` of ``pairs``: one
-    launch (``mlpmk_convert``) where every pair is contiguous, on ``dev`` and
-    of a type the library knows, else torch operations.  The destinations are
+    launch for 16 of them (``mlpmk_convert``) where every pair is contiguous,
+    on ``dev`` and of a type the library knows, else torch operations.  The destinations are
     fresh contiguous tensors of the caller."""
     if not pairs:
         return
-    if len(pairs) <= 16 and dev.type == "cuda":
+    if dev.type == "cuda":
         items = []
         for s, d in pairs:
             if not _convertible(s, dev) or d.dtype not in _CODES or d.numel() >= 1 << 31:
@@ -285,7 +286,12 @@ def as_inputs(x, weights, dt, pad=0):
 def _convert_raw(dev, items):
     """``mlpmk_convert`` of ``items``: 8 ints per matrix (source pointer and
     type, destination pointer and type, source rows and columns, destination
-    rows and columns)."""
+    rows and columns), in as many launches as their number takes."""
+    for i in range(0, len(items), 8 * _MAX_CONVERT):
+        _convert_some(dev, items[i : i + 8 * _MAX_CONVERT])
+
+
+def _convert_some(dev, items):
     f = _fast()
     if f is not None:
         rc = _launch(dev, f.convert, items)

@@ -89,3 +89,50 @@ def test_padded_module_gradients_have_the_parameters_types():
         for g, r in zip(got, want):
             assert g.dtype == dt and g.shape == r.shape
             assert ((g.double() - r).norm() / r.norm()).item() < 1e-2
+
+
+def test_more_matrices_than_one_call_takes_go_in_several(monkeypatch):
+    calls = []
+
+    def launch(dev, fn, *args):
+        calls.append(len(args[0]) // 8 if isinstance(args[0], list) else args[0])
+        return 0
+
+    monkeypatch.setattr(ops, "_launch", launch)
+    items = [v for i in range(35) for v in (A, 0, A, 1, 4, 4, 4, 4)]
+    ops._convert_raw(torch.device("cuda", 0), items)
+    assert calls == [16, 16, 3]
+    ops._convert_raw(torch.device("cuda", 0), [])
+    assert len(calls) == 3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layers", [16, 17, 33])
+def test_deep_16_bit_modules_train(layers, dt):
+    # one gradient per layer to convert: more of them than one call takes
+    import fused_mlp
+
+    torch.manual_seed(layers)
+    model = fused_mlp.FusedMLPSoftplus(D=24, H=32, out_features=8, n_layers=layers).cuda()
+    with torch.no_grad():
+        for w in model.weights:
+            w *= 1.5  # gradients of every layer between 1e-2 and 1e4: normal in both types
+    model.to(dt)
+    x = torch.randn(129, 24, device="cuda").to(dt).requires_grad_()
+    out = model(x)
+    got = torch.autograd.grad(out, [x, *model.weights], torch.ones_like(out))
+    ws = [w.detach().double().requires_grad_() for w in model.weights]
+    xs = x.detach().double().requires_grad_()
+    a = xs
+    for i, w in enumerate(ws):
+        a = a @ w
+        if i + 1 < layers:
+            h = torch.nn.functional.softplus(a)
+            a = h + (h.to(dt).double() - h).detach()  # rounded between layers, as the network rounds it
+    want = torch.autograd.grad(a, [xs, *ws], torch.ones_like(a))
+    # each layer's data gradient is rounded to dt once: 2^-11 (2^-8) a layer
+    tol = 4 * layers ** 0.5 * (2.0 ** -11 if dt == torch.float16 else 2.0 ** -8)
+    for g, r in zip(got, want):
+        assert g.dtype == dt and g.shape == r.shape
+        assert ((g.double() - r).norm() / r.norm()).item() <= tol
