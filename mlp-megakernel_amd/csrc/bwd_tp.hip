@@ -324,9 +324,10 @@ struct DgWave {
         __builtin_amdgcn_sched_barrier(0);
       }
     } else {
-      // Whole turns of kRing K-steps: the tile holds zeros up to a multiple of
-      // 64 features.
-      const int KS = (dimw<N>(p, l + 1) + 15) / 16;
+      // Whole turns of kRing K-steps: past the true width both the tile and the
+      // fragments hold zeros up to a multiple of 64 features.  (Zero fragments
+      // alone are not enough: an infinite dz would meet them as inf * 0 = NaN.)
+      const int KS = pack_ks(dimw<N>(p, l + 1));
       for (int c = 0; c < KS; c += kRing) {
 #pragma unroll
         for (int t = 0; t < kRing; ++t) {
@@ -360,10 +361,13 @@ struct DgWave {
 #pragma unroll
         for (int j = 0; j < 16; ++j) v[j] = acc[b][j] * sig_from_h(h[l][b][j]);
         store_row16(dz, W, b, v);  // for the weight-gradient pass
-        if constexpr (HAND) {      // and for the next layer, through the tile (waves past the width write zeros)
+        if constexpr (HAND) {      // and for the next layer, through the tile
           if (!N::gen || 32 * w < ((W + 63) & ~63)) {
-            const Opnd lo = make_op<EM>(*reinterpret_cast<const float(*)[8]>(v));
-            const Opnd hi = make_op<EM>(*reinterpret_cast<const float(*)[8]>(v + 8));
+            Opnd lo = make_op<EM>(*reinterpret_cast<const float(*)[8]>(v));
+            Opnd hi = make_op<EM>(*reinterpret_cast<const float(*)[8]>(v + 8));
+            // (widths are multiples of 16: past them zeros, whatever the products were)
+            if (N::gen && 32 * w >= W) lo = Opnd{f16x8{}, f16x8{}};
+            if (N::gen && 32 * w + 16 >= W) hi = Opnd{f16x8{}, f16x8{}};
             tile[par][0][slot<CH>(32 * b + n, 4 * w + g)] = lo.h;
             tile[par][0][slot<CH>(32 * b + n, 4 * w + 2 + g)] = hi.h;
             if constexpr (NT == 2) {

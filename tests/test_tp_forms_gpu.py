@@ -55,3 +55,37 @@ def test_two_pass_backward_forms(dims, m, elem, how):
         dz = dh * -torch.expm1(-hs[l - 1].double()) if l > 0 else dh
     rows = dz.abs().amax(dim=1, keepdim=True)
     assert bool(((dx.double() - dz).abs() <= max(tol / 2, 2e-4) * (dz.abs() + rows)).all()), "dx"
+
+
+def _classes(t):
+    """0 finite, 1 +inf, 2 -inf, 3 NaN"""
+    return torch.isnan(t) * 3 + torch.isposinf(t) * 1 + torch.isneginf(t) * 2
+
+
+@pytest.mark.parametrize("dims,m,elem", [
+    ((80, 112, 48, 96, 24), 300, "f16"), ((16, 96, 80, 8), 5000, "bf16"), ((64, 80, 40), 33, "f16"),
+    ((144, 208, 16, 256, 136), 1000, "f16"), ((96, 160, 104), 20000, "bf16"),       # weights as they are
+    ((144, 208, 176, 136), 40001, "f16"), ((96, 160, 104), 32768, "bf16"),          # packed
+])
+def test_an_infinite_output_gradient_stays_infinite(dims, m, elem):
+    # Weights and activations of one sign: dL/dout = inf in one place gives inf
+    # everywhere it reaches and NaN nowhere.  The K-steps that pad a layer's
+    # features to whole turns must add nothing to that.
+    dt = {"f16": torch.float16, "bf16": torch.bfloat16}[elem]
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x = (torch.rand((m, dims[0]), generator=g, device="cuda") + 0.1).to(dt)
+    ws = [((torch.rand(s, generator=g, device="cuda") + 0.5) / s[0]).to(dt) for s in zip(dims, dims[1:])]
+    _, hs = ops.fwd(x, ws, stash=True)
+    dout = (torch.rand((m, dims[-1]), generator=g, device="cuda") + 0.1).to(dt)
+    dout[m // 2, 3], dout[m - 1, 6] = float("inf"), float("-inf")
+    dws = [torch.full(tuple(w.shape), float("nan"), device="cuda") for w in ws]
+    dx = torch.empty_like(x)
+    ops.bwd(x, ws, hs, dout, dws, dx, accumulate=False)
+    want = torch.zeros((m, 1), dtype=torch.long, device="cuda")
+    want[m // 2], want[m - 1] = 1, 2
+    assert torch.equal(_classes(dx), want.expand(m, dims[0]))
+    top = torch.zeros(dims[-1], dtype=torch.long, device="cuda")
+    top[3], top[6] = 1, 2
+    assert torch.equal(_classes(dws[-1]), top.expand(dims[-2], dims[-1]))
+    for d in dws[:-1]:  # +inf of one row and -inf of the other meet
+        assert torch.isnan(d).all()
