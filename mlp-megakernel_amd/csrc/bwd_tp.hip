@@ -231,21 +231,22 @@ struct DgWave {
     const int64_t str = st > 0 ? st : 0;
     const uint32_t bytes = !nr ? 0u : scalar ? (uint32_t)kEs<EM> : (uint32_t)(((nr - 1) * str + OW) * kEs<EM>);
     const rsrc_t r = make_rsrc(static_cast<const char*>(p.dout) + row0 * str * kEs<EM>, bytes);
+    const uint32_t past = bytes;  // (not kPast: rows of a wide gradient may lie more than 2 GiB apart)
 #pragma unroll
     for (int k = 0; k < PD; ++k) {
       const int q = (int)threadIdx.x + k * G::NWV * 64, row = q / OCH, c = 8 * (q % OCH);
       const bool ok = (uint32_t)row < nr && c < OW;
       if (scalar) {
         if constexpr (EM == EM_F32) {
-          const float v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, ok ? 0 : (int)kPast, 0, 0));
+          const float v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, ok ? 0 : (int)past, 0, 0));
           dr[k].v[0] = dr[k].v[NT - 1] = f32x4{v, v, v, v};
         } else {
-          const int v = (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(r, ok ? 0 : (int)kPast, 0, 0);
+          const int v = (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(r, ok ? 0 : (int)past, 0, 0);
           const int vv = v | (v << 16);
           dr[k].v[0] = __builtin_bit_cast(f32x4, (i32x4){vv, vv, vv, vv});
         }
       } else {
-        dr[k] = load_raw(r, ok ? (uint32_t)(row * str + c) * kEs<EM> : kPast);
+        dr[k] = load_raw(r, ok ? (uint32_t)(row * str + c) * kEs<EM> : past);
       }
     }
   }

@@ -89,3 +89,27 @@ def test_an_infinite_output_gradient_stays_infinite(dims, m, elem):
     assert torch.equal(_classes(dws[-1]), top.expand(dims[-2], dims[-1]))
     for d in dws[:-1]:  # +inf of one row and -inf of the other meet
         assert torch.isnan(d).all()
+
+
+@pytest.mark.parametrize("elem", ["f16", "f32"])
+def test_output_gradient_rows_more_than_2_gib_apart(elem):
+    # A column slice of a very wide gradient: the rows of a tile span more than
+    # 2^31 bytes, and what lies between them (NaN here) is never an operand.
+    dt, dims, m = (torch.float16, (144, 208, 72), 32) if elem == "f16" else (torch.float32, (80, 112, 72), 32)
+    es = 2 if elem == "f16" else 4
+    stride = (1 << 31) // (31 * es) // 8 * 8 + 4096
+    g = torch.Generator(device="cuda").manual_seed(0)
+    x = torch.randn((m, dims[0]), generator=g, device="cuda").to(dt)
+    ws = [(torch.randn(s, generator=g, device="cuda") / s[0] ** 0.5).to(dt) for s in zip(dims, dims[1:])]
+    _, hs = ops.fwd(x, ws, stash=True)
+    dout = torch.randn((m, dims[-1]), generator=g, device="cuda").to(dt)
+    far = torch.full((m * stride,), float("nan"), dtype=dt, device="cuda").as_strided((m, dims[-1]), (stride, 1))
+    far.copy_(dout)
+    res = []
+    for d in (dout, far):
+        dws = [torch.zeros(tuple(w.shape), device="cuda") for w in ws]
+        dx = torch.empty_like(x)
+        ops.bwd(x, ws, hs, d, dws, dx)
+        res.append([dx, *dws])
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
