@@ -83,7 +83,7 @@ def _layers_workspace(dims, dtype):
     n = _layers_ws.get(key)
     if n is None:
         out = ctypes.c_int64(-1)
-        if dtype != torch.float32:
+        if dtype != torch.float32 and min(dims) > 0:  # (a layer of no features is the library GEMMs' to run)
             rc = _lib.get().mlpmk_fwd_layers_workspace_size(len(dims) - 1, _lib.dims_array(dims), _fwd_code(dtype),
                                                             ctypes.byref(out))
             if rc not in (0, 2):  # MLPMK_ERR_UNSUPPORTED_SHAPE: -1 stays

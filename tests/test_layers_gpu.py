@@ -181,3 +181,30 @@ def test_infinities_stay_where_the_oracle_has_them(dims, elem):
         fin[150] = False
         ok, err, _ = orc.allclose_report(got[fin], want[fin], 1e-2 if elem == "f16" else 3e-2, 1e-2 if elem == "f16" else 3e-2)
         assert ok, err
+
+
+def test_empty_widths_are_left_to_the_library_route():
+    # a layer of no features is no network of this kernel, and no error either
+    for dims in ((16, 0, 8), (0, 320, 8), (16, 320, 0)):
+        assert fallback._layers_workspace(dims, torch.float16) == -1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims", [(16, 0, 8), (0, 320, 8), (16, 320, 0), (5, 0, 0, 4)])
+def test_networks_with_an_empty_layer_run(dims):
+    from mlpmk.autograd import fused_mlp
+
+    g = torch.Generator(device="cuda").manual_seed(0)
+    x = torch.randn((9, dims[0]), generator=g, device="cuda").half().requires_grad_()
+    ws = [torch.randn(s, generator=g, device="cuda").half().requires_grad_() for s in zip(dims, dims[1:])]
+    out = fused_mlp(x, *ws)
+    ref = x.double()
+    for i, w in enumerate(ws):
+        ref = ref @ w.double()
+        ref = torch.nn.functional.softplus(ref) if i + 1 < len(ws) else ref
+    torch.testing.assert_close(out.double(), ref, atol=1e-1, rtol=1e-2)
+    grads = torch.autograd.grad(out.sum(), [x, *ws])
+    want = torch.autograd.grad(ref.sum(), [x, *ws])
+    for got, r in zip(grads, want):
+        assert got.dtype == torch.float16 and got.shape == r.shape
+        torch.testing.assert_close(got.double(), r.double(), atol=1e-1, rtol=2e-2)
