@@ -208,3 +208,24 @@ def test_networks_with_an_empty_layer_run(dims):
     for got, r in zip(grads, want):
         assert got.dtype == torch.float16 and got.shape == r.shape
         torch.testing.assert_close(got.double(), r.double(), atol=1e-1, rtol=2e-2)
+
+
+@pytest.mark.gpu
+def test_layers_softplus_keeps_its_digits_over_the_whole_range():
+    # z = x w exactly, as above, down to where e^z leaves the normal fp32 range
+    # (-87.3) and up past the threshold of 20, at fp16 steps.  The two-part
+    # product leaves e^z with the roundings of the exponential (1 ulp), of the
+    # correction and of the sum: 4 ulp of 2^-23 in all, as in the elementwise
+    # kernel of the layer-by-layer path, which is held to the same bound.
+    z = torch.cat([torch.linspace(-87, 24, 4096), torch.linspace(-1.5, 1.5, 4096)]).half().reshape(16, 512)
+    for part in z.cuda():
+        x = torch.zeros((4, 8), device="cuda", dtype=torch.float16)
+        x[:, 0] = 1
+        w0 = torch.zeros((8, 512), device="cuda", dtype=torch.float16)
+        w0[0] = part
+        _, (h,) = fallback._fwd_layers(x, [w0, torch.zeros((512, 8), device="cuda", dtype=torch.float16)], True)
+        d = part.double()
+        ref = torch.clamp(d, min=0) + torch.log1p(torch.exp(-d.abs()))
+        for name, got in (("fwd_layers", h[0]), ("softplus_f32", fallback.softplus_f32(part.float()))):
+            err = ((got.double() - ref).abs() / ref).max().item()
+            assert err <= 4 * 2.0 ** -23, (name, part[0].item(), part[-1].item(), err)
