@@ -269,15 +269,26 @@ def as_inputs(x, weights, dt, pad=0):
     todo, res = [], []
     for i, t in enumerate([x] + weights):
         p = pad if i < 2 else 0
+        if not t.is_contiguous():
+            # Cast while it is gathered: in row order in its own type first, a
+            # transposed fp32 x of 524,288 x 128 took 574 us with the network
+            # behind it, not 335 (a column slice 223, not 133).
+            if p and t.dim() == 2:
+                d = torch.zeros((t.shape[0], t.shape[1] + p) if i == 0 else (t.shape[0] + p, t.shape[1]), dtype=dt,
+                                device=t.device)
+                d[: t.shape[0], : t.shape[1]].copy_(t)
+                res.append(d)
+                continue
+            t = t.to(dt).contiguous()
         if t.dtype == dt and not p:
-            res.append(t.contiguous())
+            res.append(t)
             continue
         if t.dim() != 2:  # (the callers' own checks name it)
-            res.append(t.to(dt).contiguous())
+            res.append(t.to(dt))
             continue
         rows, cols = int(t.shape[0]), int(t.shape[1])
         d = torch.empty((rows, cols + p) if i == 0 else (rows + p, cols), dtype=dt, device=t.device)
-        todo.append((t.contiguous(), d))
+        todo.append((t, d))
         res.append(d)
     convert(todo, x.device)
     return res[0], res[1:]

@@ -136,3 +136,21 @@ def test_deep_16_bit_modules_train(layers, dt):
     for g, r in zip(got, want):
         assert g.dtype == dt and g.shape == r.shape
         assert ((g.double() - r).norm() / r.norm()).item() <= tol
+
+
+@pytest.mark.parametrize("pad", [0, 13])
+@pytest.mark.parametrize("layout", ["rows", "transposed", "slice", "expanded"])
+def test_strided_inputs_are_cast_while_they_are_gathered(monkeypatch, layout, pad):
+    g = torch.Generator().manual_seed(0)
+    x = {"rows": lambda: torch.randn((40, 3), generator=g), "transposed": lambda: torch.randn((3, 40), generator=g).t(),
+         "slice": lambda: torch.randn((40, 9), generator=g)[:, 2:5],
+         "expanded": lambda: torch.randn((1, 3), generator=g).expand(40, 3)}[layout]()
+    w = torch.randn((3, 16), generator=g)
+    seen, convert = [], ops.convert
+    monkeypatch.setattr(ops, "convert", lambda pairs, dev: (seen.extend(s for s, _ in pairs), convert(pairs, dev)))
+    xc, (wc,) = ops.as_inputs(x, [w], torch.float16, pad)
+    assert xc.is_contiguous() and wc.is_contiguous()
+    assert torch.equal(xc, torch.nn.functional.pad(x, (0, pad)).half())
+    assert torch.equal(wc, torch.nn.functional.pad(w, (0, 0, 0, pad)).half())
+    # only what lies in rows reaches the conversion launch
+    assert [s.data_ptr() for s in seen] == ([x.data_ptr()] if layout == "rows" else []) + [w.data_ptr()]
