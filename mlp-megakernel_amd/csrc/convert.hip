@@ -48,20 +48,32 @@ __global__ __launch_bounds__(256) void convert_kernel(Params p) {
   float v[8] = {};
   if (t.raw && !(t.vec && e + 8 <= have)) {
     const uint16_t* s = static_cast<const uint16_t*>(t.src);
-    uint16_t* d = static_cast<uint16_t*>(t.dst);
     uint32_t r = e / t.dst_cols, c = e - r * t.dst_cols;
-    uint16_t b[8];
+    typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+    u16x8 b = {};
+    if (t.dst_cols % 8 == 0 && r < t.src_rows && c + 8 <= t.src_cols) {
+      // Padding to whole pieces (every caller's): eight elements of one row, at
+      // any element boundary of the source, in one load.  Element by element in
+      // and out, 524,288 x 63 bf16 into 64 columns took 53 us, this way 29 (fp32 56 and 44).
+      __builtin_memcpy(&b, s + r * t.src_cols + c, 16);
+    } else {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      b[j] = r < t.src_rows && c < t.src_cols ? s[r * t.src_cols + c] : (uint16_t)0;
-      if (++c == t.dst_cols) {
-        c = 0;
-        ++r;
+      for (int j = 0; j < 8; ++j) {
+        if (r < t.src_rows && c < t.src_cols) b[j] = s[r * t.src_cols + c];
+        if (++c == t.dst_cols) {
+          c = 0;
+          ++r;
+        }
       }
     }
+    uint16_t* d = static_cast<uint16_t*>(t.dst);
+    if (e + 8 <= t.n) {  // dst is 16-byte aligned
+      reinterpret_cast<u16x8*>(d)[e / 8] = b;
+    } else {
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (e + j < t.n) d[e + j] = b[j];
+      for (int j = 0; j < 8; ++j)
+        if (e + j < t.n) d[e + j] = b[j];
+    }
     return;
   }
   if (t.flat) {
@@ -90,12 +102,16 @@ __global__ __launch_bounds__(256) void convert_kernel(Params p) {
     }
   } else {
     uint32_t r = e / t.dst_cols, c = e - r * t.dst_cols;
+    if (t.src_dt == MLPMK_DTYPE_F32 && t.dst_cols % 8 == 0 && r < t.src_rows && c + 8 <= t.src_cols) {
+      __builtin_memcpy(v, static_cast<const float*>(t.src) + r * t.src_cols + c, 32);
+    } else {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (r < t.src_rows && c < t.src_cols) v[j] = load1(t.src, r * t.src_cols + c, t.src_dt);
-      if (++c == t.dst_cols) {
-        c = 0;
-        ++r;
+      for (int j = 0; j < 8; ++j) {
+        if (r < t.src_rows && c < t.src_cols) v[j] = load1(t.src, r * t.src_cols + c, t.src_dt);
+        if (++c == t.dst_cols) {
+          c = 0;
+          ++r;
+        }
       }
     }
   }

@@ -154,3 +154,24 @@ def test_strided_inputs_are_cast_while_they_are_gathered(monkeypatch, layout, pa
     assert torch.equal(wc, torch.nn.functional.pad(w, (0, 0, 0, pad)).half())
     # only what lies in rows reaches the conversion launch
     assert [s.data_ptr() for s in seen] == ([x.data_ptr()] if layout == "rows" else []) + [w.data_ptr()]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sd,dd", list(itertools.product(TYPES, TYPES)))
+@pytest.mark.parametrize("off", [0, 1, 3])
+def test_padding_to_whole_pieces_from_any_element_boundary(sd, dd, off):
+    # pieces of eight that lie in the row, straddle its end, or lie past it or
+    # past the last row, from sources that start off a 16-byte boundary
+    g = torch.Generator(device="cuda").manual_seed(off)
+    view = torch.int32 if dd == torch.float32 else torch.int16
+    pairs = []
+    for (r, c), (dr, dc) in [((301, 63), (301, 64)), ((70, 13), (70, 16)), ((3, 8), (5, 16)), ((9, 7), (9, 8)),
+                             ((40, 24), (41, 24)), ((17, 100), (20, 112)), ((33, 21), (30, 16)), ((6, 17), (6, 20))]:
+        src = torch.randn(off + r * c, generator=g, device="cuda").to(sd)[off:].view(r, c)
+        pairs.append((src, torch.full((dr, dc), 7.0, dtype=dd, device="cuda")))
+    ops.convert(pairs, pairs[0][0].device)
+    for s, d in pairs:
+        ref = torch.zeros_like(d)
+        r, c = min(s.shape[0], d.shape[0]), min(s.shape[1], d.shape[1])
+        ref[:r, :c] = s[:r, :c].to(dd)
+        assert torch.equal(d.view(view), ref.view(view)), (s.shape, d.shape)
