@@ -92,19 +92,39 @@ def _layers_workspace(dims, dtype):
     return n
 
 
+def _gemms_faster(dims, M):
+    """True where the library GEMMs run a narrow 16-bit network sooner than the
+    one-launch kernel.  That kernel spends 0.12 ns per row on each layer of at
+    most 64 features, whatever their number (6 of its 8 waves have no feature
+    group); the GEMM route moves about 28 bytes per row and hidden feature and
+    10 per input and output feature, at 2 to 4 TB/s from a few hundred
+    thousand rows on (below, its launches take longer: 38 us a layer).
+    Kernel / GEMMs in us, bytes per layer in brackets: 8-8-1 [157] 350,000 rows
+    99 / 83, 1,200,000 318 / 210; 8-8-8-8 [203] 350,000 136 / 138, 500,000 189 /
+    172, 1,200,000 443 / 350; 24-8-8-24 [309] 500,000 193 / 245, 2,097,152 772 /
+    700; 63-8-8-1 [363] 2,097,152 1042 / 737; 7 x 16 [427] 500,000 383 / 426,
+    2,097,152 1561 / 1535; 16-24-16 [496] 1,048,576 257 / 270, 4,194,304 1007 /
+    1126."""
+    if M < 400000:
+        return False
+    moved = 10 * (dims[0] + dims[-1]) + 28 * sum(dims[1:-1])
+    return moved < (400 if M >= 1 << 20 else 300) * (len(dims) - 1)
+
+
 def _fwd_layers(x, weights, stash):
     """:func:`fwd` through ``mlpmk_fwd_layers``, or None where that kernel does
     not take the call (fp32 tensors, widths above 512, more than 8 layers,
     hidden widths that are not multiples of 8, tensors off a 16-byte
-    boundary).  An input width that is not a multiple of 8 is padded with zero
-    columns of x and zero rows of W_1, which add nothing to the product."""
+    boundary) or is not the faster route (``_gemms_faster``).  An input width
+    that is not a multiple of 8 is padded with zero columns of x and zero rows
+    of W_1, which add nothing to the product."""
     if x.dim() != 2 or any(w.dim() != 2 for w in weights):
         return None
     dims = (int(x.shape[1]),) + tuple(int(w.shape[1]) for w in weights)
+    if x.device.type != "cuda" or any(w.device != x.device for w in weights) or _gemms_faster(dims, int(x.shape[0])):
+        return None
     pad = -dims[0] % 8
     dims = (dims[0] + pad,) + dims[1:]
-    if x.device.type != "cuda" or any(w.device != x.device for w in weights):
-        return None
     nbytes = _layers_workspace(dims, x.dtype)
     if nbytes < 0 or any(tuple(w.shape) != (k, n) for w, k, n in zip(weights, (dims[0] - pad,) + dims[1:], dims[1:])):
         return None

@@ -229,3 +229,28 @@ def test_layers_softplus_keeps_its_digits_over_the_whole_range():
         for name, got in (("fwd_layers", h[0]), ("softplus_f32", fallback.softplus_f32(part.float()))):
             err = ((got.double() - ref).abs() / ref).max().item()
             assert err <= 4 * 2.0 ** -23, (name, part[0].item(), part[-1].item(), err)
+
+
+@pytest.mark.parametrize("dims,m,gemms", [
+    ((8, 8, 1), 399999, False), ((8, 8, 1), 400000, True), ((8, 8, 8, 8), 400000, True), ((16, 8, 16), 400000, True),
+    ((24, 8, 8, 24), 1048575, False), ((24, 8, 8, 24), 1048576, True), ((63, 8, 8, 1), 1048576, True),
+    ((16,) * 7, 4194304, False), ((16, 24, 16), 4194304, False), ((128, 512, 512, 128), 1048576, False),
+])
+def test_narrow_networks_of_many_rows_go_to_the_gemms(dims, m, gemms):
+    assert fallback._gemms_faster(dims, m) is gemms
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims", [(8, 8, 1), (3, 8, 8, 16)])
+def test_both_routes_of_a_narrow_network_agree(dims):
+    m = 400000
+    x, ws = orc.make_inputs(dims, m, seed=1)
+    xd, wd = torch.from_numpy(x).cuda(), [torch.from_numpy(w).cuda() for w in ws]
+    assert fallback._fwd_layers(xd, wd, True) is None
+    out, hs = fallback.fwd(xd, wd, stash=True)
+    part, phs = fallback._fwd_layers(xd[: m - 1], wd, True)
+    # fp32 accumulation and softplus on both routes: the stash within a few fp32
+    # ulp of the largest terms, an output element within a rounding of h and out
+    torch.testing.assert_close(out[: m - 1], part, atol=2.0 ** -9, rtol=2.0 ** -9)
+    torch.testing.assert_close(hs[0][: m - 1], phs[0], atol=2e-6, rtol=2e-6)
+    assert all(h.shape == (m, d) and h.dtype == torch.float32 for h, d in zip(hs, dims[1:]))
