@@ -816,13 +816,16 @@ int launch_dgrad(const TpParams& p, int cus, hipStream_t st) {
 // 3x128 fp32 at 16,384 23 / 30, 32,768 35 / 34, 49,152 50 / 43 (4-wave 128 x
 // 128 at 65,536: 60, WG_PAIR 46: half the atomics, 23 us of the 60).  Below 64
 // features a 128 x 128 block is mostly empty: 3x64 fp32 32 / 32 at 65,536.
+// 16-bit networks up to 128 wide keep WG_QUAD: they come here up to 16,384 rows
+// only (bwd_path), so WG_PAIR is built for fp32 tensors and WG_WIDE for the
+// runtime-width networks of 16-bit ones.
 enum { WG_QUAD, WG_PAIR, WG_WIDE };
 constexpr int kPairMinRows = 32768, kWideMinRows = 24576;
-int wgrad_form(int L, const int* dims, int64_t M) {
+int wgrad_form(int L, const int* dims, int64_t M, bool f32) {
   int wmax = 0;
   for (int i = 0; i <= L; ++i) wmax = dims[i] > wmax ? dims[i] : wmax;
   if (wmax > 128) return M >= kWideMinRows ? WG_WIDE : WG_QUAD;
-  return wmax > 64 && M >= kPairMinRows ? WG_PAIR : WG_QUAD;
+  return f32 && wmax > 64 && M >= kPairMinRows ? WG_PAIR : WG_QUAD;
 }
 
 int quad_blocks(int L, const int* dims, int form) {
@@ -849,7 +852,7 @@ constexpr int64_t kF32MaxChunkRows = 8192;
 // many chunks with the passes spread evenly -- and with fp32 tensors of at
 // most kF32MaxChunkRows rows.
 int wgrad_chunks(int L, const int* dims, int64_t M, bool f32, int cus) {
-  const int form = wgrad_form(L, dims, M);
+  const int form = wgrad_form(L, dims, M, f32);
   const int rp = (form == WG_QUAD ? 256 : 128) / (f32 ? 2 : 1);  // rows per pass (WgGeo::RP)
   const int nqb = quad_blocks(L, dims, form);
   const int64_t passes = (M + rp - 1) / rp;
@@ -872,10 +875,11 @@ int launch_wgrad(const TpParams& p, int S, int nqb, hipStream_t st) {
 
 template <class N, int EM>
 int launch_wgrad_form(const TpParams& p, int form, int S, int nqb, int cus, hipStream_t st) {
-  if constexpr (EM != tp::EM_F32) {
+  if constexpr (EM == tp::EM_F32) {
+    if (form == WG_PAIR) return launch_wgrad<N, EM, 2, 2, 2, 1>(p, S, nqb, st);
+  } else if constexpr (N::gen) {
     if (form == WG_WIDE) return launch_wgrad<N, EM, 2, 4, 1, 1>(p, S, nqb, st);
   }
-  if (form == WG_PAIR) return launch_wgrad<N, EM, 2, 2, 2, 1>(p, S, nqb, st);
   return (int64_t)S * nqb > cus ? launch_wgrad<N, EM, 1, 1, 1, 2>(p, S, nqb, st)
                                 : launch_wgrad<N, EM, 1, 1, 1, 1>(p, S, nqb, st);
 }
@@ -929,7 +933,7 @@ int dispatch_l(const TpParams& p, const int* dims, int S, hipStream_t st) {
   if (rc != MLPMK_OK) return rc;
   // Pass 2 (the kernel reads only N's layer count and whether its widths are
   // fixed: one runtime-width instance per depth serves every shape).
-  const int form = wgrad_form(L, dims, p.M);
+  const int form = wgrad_form(L, dims, p.M, EM == tp::EM_F32);
   const int nqb = quad_blocks(L, dims, form);
   typedef typename GenTp<L>::W NW;
   rc = L == 3 && is_3l128(L, dims) ? launch_wgrad_form<TNet3L128, EM>(p, form, S, nqb, cus, st)
