@@ -24,6 +24,10 @@ CASES = [
     # data-gradient tiles: 32 rows up to 16,384, 64 from there
     ((128, 256, 256, 128), 16384, "f16"), ((128, 256, 256, 128), 16385, "f16"), ((96, 160, 104), 3, "f16"),
     ((128, 128, 128, 128), 33, "f16"), ((64, 128, 64, 32, 128, 120), 16449, "f32"),
+    # weights read in place below 32,768 rows, packed first from there
+    ((128, 256, 256, 128), 32767, "bf16"), ((128, 256, 256, 128), 32768, "bf16"), ((144, 208, 72), 32768, "f16"),
+    ((96, 160, 104), 33011, "bf16"), ((144, 176, 208, 136), 33011, "bf16"), ((256, 256, 256, 8), 32769, "f16"),
+    ((16, 144, 144, 144, 144, 72), 32768, "bf16"), ((176, 256, 16, 256, 144, 136), 33011, "f16"),
 ]
 
 
@@ -113,3 +117,38 @@ def test_output_gradient_rows_more_than_2_gib_apart(elem):
         res.append([dx, *dws])
     for a, b in zip(*res):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dims,m,elem", [((144, 176, 208, 136), 33011, "bf16"), ((128, 256, 256, 128), 32768, "f16"),
+                                         ((96, 160, 104), 40001, "f16"), ((16, 144, 144, 144, 144, 72), 32768, "bf16")])
+def test_a_workspace_without_room_for_the_packed_weights_serves(dims, m, elem):
+    # Both forms at one batch: the same fragments in the same order give the
+    # bits of dx; dW differs by the order of its atomics only.
+    from mlpmk import _lib
+
+    dt = {"f16": torch.float16, "bf16": torch.bfloat16}[elem]
+    L = len(dims) - 1
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.randn((m, dims[0]), generator=g, device="cuda").to(dt)
+    ws = [(torch.randn(s, generator=g, device="cuda") / s[0] ** 0.5).to(dt) for s in zip(dims, dims[1:])]
+    _, hs = ops.fwd(x, ws, stash=True)
+    dout = torch.randn((m, dims[-1]), generator=g, device="cuda").to(dt)
+    need = ops.bwd_workspace_bytes(dims, m, True, dtype=dt)
+    packed = sum(-(-k // 32) * (-(-n // 64) * 4) * 1024 for k, n in zip(dims, dims[1:]))
+    lib, dev = _lib.get(), x.device
+    buf = torch.empty(need, dtype=torch.uint8, device="cuda")
+    res = []
+    for nbytes, want in ((need, 0), (need - packed, 0), (need - packed - 256, 1)):
+        dws = [torch.zeros(tuple(w.shape), device="cuda") for w in ws]
+        dx = torch.full_like(x, float("nan"))
+        buf[nbytes:] = 0xA5
+        arr = lambda ts: (_lib.c_void_p * len(ts))(*[t.data_ptr() for t in ts])  # noqa: E731
+        rc = ops._launch(dev, lib.mlpmk_bwd_ws, L, _lib.dims_array(dims), ops._fwd_code(dt), x.data_ptr(), arr(ws),
+                         arr(hs), dout.data_ptr(), dims[-1], dx.data_ptr(), arr(dws), buf.data_ptr(), nbytes, m)
+        torch.cuda.synchronize()
+        assert rc == want and bool((buf[nbytes:] == 0xA5).all())
+        if rc == 0:
+            res.append((dx, dws))
+    assert torch.equal(res[0][0], res[1][0]) and bool(torch.isfinite(res[0][0]).all())
+    for a, b in zip(res[0][1], res[1][1]):
+        assert ((a - b).norm() / a.norm()).item() < 1e-5  # fp32 sums in another order
