@@ -24,6 +24,11 @@ CASES = [
     # data-gradient tiles: 32 rows up to 16,384, 64 from there
     ((128, 256, 256, 128), 16384, "f16"), ((128, 256, 256, 128), 16385, "f16"), ((96, 160, 104), 3, "f16"),
     ((128, 128, 128, 128), 33, "f16"), ((64, 128, 64, 32, 128, 120), 16449, "f32"),
+    # tiles of 32 and 64 rows by the rows that the CU with most gets, by the
+    # hidden widths, and with resident weights
+    ((128, 128, 128, 128), 131071, "f32"), ((128, 128, 128, 128), 131073, "f32"), ((32, 96, 96, 16), 20000, "f32"),
+    ((32, 96, 96, 16), 24577, "f32"), ((16, 128, 128, 24), 16385, "f32"), ((16, 144, 144, 72), 24576, "bf16"),
+    ((16, 144, 144, 72), 24577, "bf16"), ((64, 192, 208, 40), 16385, "f16"),
     # weights read in place below 32,768 rows, packed first from there
     ((128, 256, 256, 128), 32767, "bf16"), ((128, 256, 256, 128), 32768, "bf16"), ((144, 208, 72), 32768, "f16"),
     ((96, 160, 104), 33011, "bf16"), ((144, 176, 208, 136), 33011, "bf16"), ((256, 256, 256, 8), 32769, "f16"),
