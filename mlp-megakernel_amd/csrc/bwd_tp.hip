@@ -795,12 +795,12 @@ int launch_dgrad_rb(const TpParams& p, int cus, hipStream_t st) {
 // Tiles of 64 rows read the weights once for twice the rows, but hand a CU its
 // rows in twice as large steps: at 20,000 rows two of them (128 rows) where
 // tiles of 32 make three (96).  So 64 rows from 64 rows per CU on where that is
-// no more rows for the CU with most, or where the weights weigh more: hidden
+// at most 7 % more rows for the CU with most, or where the weights weigh more: hidden
 // widths of 128 with fp32 tensors, of 192 and more in 16 bits.  With resident
 // weights (RES) nothing is read again, and 64 rows pay from 512 per CU on.
 // Whole backward, us, tiles of 64 / 32 rows: 3x128 fp32 20,000 rows 47 / 43,
 // 65,536 85 / 83, 131,072 155 / 160, 600,000 642 / 667; 32-96-96-96-16 fp32 24,000
-// 49 / 45, 131,072 175 / 192; 5x128 fp32 24,000 85 / 87, 32,768 87 / 98;
+// 49 / 45, 131,072 175 / 192, 200,003 278 / 301; 5x128 fp32 24,000 85 / 87, 32,768 87 / 98;
 // 16-144-144-144-144-72 bf16 20,000 with dx 88 / 75; 256-256-256-256 fp16 20,000
 // 86 / 90; 4x160 fp16 17,000 66 / 64, 28,000 68 / 72.
 template <int EM, bool RES>
@@ -811,7 +811,7 @@ bool dgrad_wide_tiles(const TpParams& p, int L, int cus) {
   for (int l = 2; l < L; ++l) hidden = p.dims[l] < hidden ? p.dims[l] : hidden;
   if (hidden >= (EM == tp::EM_F32 ? 128 : 192)) return true;
   auto rounds = [&](int64_t rows) { return ((p.M + rows - 1) / rows + cus - 1) / cus; };
-  return 2 * rounds(64) <= rounds(32);
+  return 200 * rounds(64) <= 107 * rounds(32);
 }
 
 template <class N, int EM, bool DX, bool RES>
