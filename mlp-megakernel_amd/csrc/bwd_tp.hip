@@ -830,30 +830,40 @@ int launch_dgrad(const TpParams& p, int cus, hipStream_t st) {
 // blocks, 8 waves (16-bit tensors of widths above 128: the fp32 activations
 // read once, dz twice).
 //
-// Where the lines lie (this pass alone, us; QUAD / the other form):
-// 128-256-256-128 bf16 at 4,096 rows 11 / 23, 16,384 23 / 33, 32,768 39 / 45,
-// 49,152 54 / 52, 100,003 155 / 91 (4-wave 128 x 128 blocks, which WG_WIDE
-// replaced: 19, 41, 46, 53, 113); 160-192-192-192-64 fp16 at 49,152 89 / 55.
-// 3x128 fp32 at 16,384 23 / 30, 32,768 35 / 34, 49,152 50 / 43 (4-wave 128 x
-// 128 at 65,536: 60, WG_PAIR 46: half the atomics, 23 us of the 60).  Below 64
-// features a 128 x 128 block is mostly empty: 3x64 fp32 32 / 32 at 65,536.
+// The other forms win once the rows times the 64 x 64 blocks, each of which
+// reads its rows again, reach a number that depends on the chunks S of
+// WG_QUAD: where S is a multiple of the 8 XCDs, the blocks of a chunk run on
+// one XCD and share its rows in that L2, and WG_QUAD holds out 2.5 times as
+// long.  Whole backward, us, QUAD / WIDE (16-bit tensors; blocks, S):
+// 256-256-256-256 [48, 10] 12,288 rows 62 / 63, 24,000 98 / 82; 6 x 256 [80, 6]
+// 8,192 68 / 65, 24,000 172 / 123; 160-192-192-192-64 [30, 17] 12,288 43 / 51,
+// 20,000 72 / 65; 256-256-8 [20, 25] 24,000 39 / 47, 40,000 59 / 58; but
+// 128-256-256-128 [32, 16] 40,000 83 / 88, 50,000 103 / 99; 64-256-64 [8, 64]
+// 100,003 78 / 84.  QUAD / PAIR (fp32 tensors, widths above 64: a block of 128 x
+// 128 is mostly empty below): 3x128 [12, 42] 32,768 60 / 58, 65,536 100 / 85;
+// 80-80-8 [6, 85] 40,000 34 / 36, 65,536 44 / 43; but 2x128 [8, 64] 80,000 69 /
+// 74, 131,072 103.5 / 102; 4x128 [16, 32] 49,152 92 / 95, 80,000 154 / 147;
+// 64-128-64 [4, 128] 200,003 112 / 123.
 // 16-bit networks up to 128 wide keep WG_QUAD: they come here up to 16,384 rows
 // only (bwd_path), so WG_PAIR is built for fp32 tensors and WG_WIDE for the
 // runtime-width networks of 16-bit ones.
 enum { WG_QUAD, WG_PAIR, WG_WIDE };
-constexpr int kPairMinRows = 32768, kWideMinRows = 24576;
-int wgrad_form(int L, const int* dims, int64_t M, bool f32) {
-  int wmax = 0;
-  for (int i = 0; i <= L; ++i) wmax = dims[i] > wmax ? dims[i] : wmax;
-  if (wmax > 128) return M >= kWideMinRows ? WG_WIDE : WG_QUAD;
-  return f32 && wmax > 64 && M >= kPairMinRows ? WG_PAIR : WG_QUAD;
-}
 
 int quad_blocks(int L, const int* dims, int form) {
   const int fa = form == WG_QUAD ? 64 : 128, fz = form == WG_QUAD ? 64 : form == WG_PAIR ? 128 : 256;
   int n = 0;
   for (int l = 0; l < L; ++l) n += ((dims[l] + fa - 1) / fa) * ((dims[l + 1] + fz - 1) / fz);
   return n;
+}
+
+constexpr int64_t kPairMinRows = 32768;
+int wgrad_form(int L, const int* dims, int64_t M, bool f32, int cus) {
+  int wmax = 0;
+  for (int i = 0; i <= L; ++i) wmax = dims[i] > wmax ? dims[i] : wmax;
+  const int quads = quad_blocks(L, dims, WG_QUAD);
+  const bool shared = 2 * cus >= quads && 2 * cus / quads % 8 == 0;
+  if (wmax > 128) return M * quads >= (shared ? 1440000 : 540000) ? WG_WIDE : WG_QUAD;
+  return f32 && wmax > 64 && M >= kPairMinRows && M * quads >= (shared ? 880000 : 360000) ? WG_PAIR : WG_QUAD;
 }
 
 // Longest row chunk with fp32 tensors.  A chunk's products of split
@@ -873,7 +883,7 @@ constexpr int64_t kF32MaxChunkRows = 8192;
 // many chunks with the passes spread evenly -- and with fp32 tensors of at
 // most kF32MaxChunkRows rows.
 int wgrad_chunks(int L, const int* dims, int64_t M, bool f32, int cus) {
-  const int form = wgrad_form(L, dims, M, f32);
+  const int form = wgrad_form(L, dims, M, f32, cus);
   const int rp = (form == WG_QUAD ? 256 : 128) / (f32 ? 2 : 1);  // rows per pass (WgGeo::RP)
   const int nqb = quad_blocks(L, dims, form);
   const int64_t passes = (M + rp - 1) / rp;
@@ -954,7 +964,7 @@ int dispatch_l(const TpParams& p, const int* dims, int S, hipStream_t st) {
   if (rc != MLPMK_OK) return rc;
   // Pass 2 (the kernel reads only N's layer count and whether its widths are
   // fixed: one runtime-width instance per depth serves every shape).
-  const int form = wgrad_form(L, dims, p.M, EM == tp::EM_F32);
+  const int form = wgrad_form(L, dims, p.M, EM == tp::EM_F32, cus);
   const int nqb = quad_blocks(L, dims, form);
   typedef typename GenTp<L>::W NW;
   rc = L == 3 && is_3l128(L, dims) ? launch_wgrad_form<TNet3L128, EM>(p, form, S, nqb, cus, st)

@@ -24,6 +24,10 @@ CASES = [
     # data-gradient tiles: 32 rows up to 16,384, 64 from there
     ((128, 256, 256, 128), 16384, "f16"), ((128, 256, 256, 128), 16385, "f16"), ((96, 160, 104), 3, "f16"),
     ((128, 128, 128, 128), 33, "f16"), ((64, 128, 64, 32, 128, 120), 16449, "f32"),
+    # weight-gradient forms by rows times blocks of 64 x 64 (48, 80, 32, 8, 20)
+    ((256, 256, 256, 256), 11249, "f16"), ((256, 256, 256, 256), 11250, "bf16"), ((256,) * 6, 6750, "f16"),
+    ((128, 256, 256, 128), 44999, "f16"), ((128, 256, 256, 128), 45000, "f16"), ((128, 128, 128), 109999, "f32"),
+    ((128, 128, 128), 110000, "f32"), ((256, 256, 8), 27003, "f16"),
     # tiles of 32 and 64 rows by the rows that the CU with most gets, by the
     # hidden widths, and with resident weights
     ((128, 128, 128, 128), 131071, "f32"), ((128, 128, 128, 128), 131073, "f32"), ((32, 96, 96, 16), 20000, "f32"),
