@@ -18,12 +18,14 @@
 //    needs no test of a width in its loop.  (Read straight from the row-major
 //    W_l, a lane's eight inputs of one feature are eight loads; at 256-wide
 //    layers these were 20 % of such a kernel's time.)  Both launches at that
-//    size: 24.7 us per call, 4.6 us of it the packing and its launch.
+//    size: 25.4 us per call, 4.4 us of it the packing.
 //  * fwd_layers_kernel: a workgroup of 8 waves owns a tile of 32 RB rows, in
 //    one LDS tile of 16-bit activations that the layers overwrite in turn.
 //    Wave f computes output features [64 f, 64 f + 64) of every row; a layer
 //    of at most 256 features splits the rows over the waves as well, so every
-//    fragment is read by one wave, or by the few that share its rows.
+//    fragment is read by one wave, or by the few that share its rows.  (Of a
+//    layer of at most 64 features two waves have work, the others wait: 0.12 ns
+//    per row and layer whatever its width.)
 //  * Softplus as max(z, 0) + log1p(e^-|z|) in fp32, handed on rounded to the
 //    tensor format as the reference rounds its h (kernel.py:110); the stash is
 //    that fp32 value.
@@ -52,7 +54,7 @@ struct Params {
 __host__ __device__ constexpr int pad64(int n) { return (n + 63) & ~63; }
 
 // softplus(z) = max(z, 0) + log1p(y), y = e^-|z|: two transcendentals and
-// eleven more operations.
+// ten more operations.
 //  * y = 2^p e^r with p = -|z| log2 e rounded and r = -|z| - p ln 2 (ln 2 in two
 //    parts), e^r = 1 + r: without r the rounding of p alone moves y by
 //    |z| 2^-24 (3.8e-6 at z = -80; the stash is fp32, and the elementwise
@@ -61,17 +63,17 @@ __host__ __device__ constexpr int pad64(int n) { return (n + 63) & ~63; }
 //    term is what the rounding of w dropped (its factor 1 / w is left out: the
 //    term is below 2^-24 where w is not close to 1), so small y keep their
 //    digits.
-// |z| is clamped where y is 0 anyway, so that -inf gives 0 and not inf - inf;
-// the maxima propagate NaN, and +inf stays +inf.  Largest relative error, here
+// y is clamped to [0, 1], which makes the NaN (inf - inf) of an infinite z 0 and
+// takes no operation of its own (the multiply-add's output modifier); a NaN z
+// comes through the maximum.  Largest relative error, here
 // / elementwise kernel / without r: 1.4e-7 / 1.9e-7 / 3.9e-6 for z in [-87, -20],
-// 2.9e-7 / 3.5e-7 / 1.1e-6 in [-20, -5], 2.7e-7 / 3.3e-7 / 4.4e-7 above.  r costs
-// 1.5 us of 128-512-512-128's 26.0 at 16,384 rows.
+// 2.9e-7 / 3.5e-7 / 1.1e-6 in [-20, -5], 2.7e-7 / 3.3e-7 / 4.4e-7 above.  r takes
+// three operations: 128-512-512-128 at 16,384 rows 24.0 -> 25.4 us.
 constexpr float kLn2Lo = -1.904654323148236e-9f;  // ln 2 - kLn2
 __device__ __forceinline__ float softplus_n(float z) {
-  const float a = __builtin_elementwise_maximum(-__builtin_fabsf(z), -200.0f);
-  const float p = a * kLog2e, e = __builtin_amdgcn_exp2f(p);
+  const float a = -__builtin_fabsf(z), p = a * kLog2e, e = __builtin_amdgcn_exp2f(p);
   const float r = __builtin_fmaf(p, -kLn2Lo, __builtin_fmaf(p, -kLn2, a));
-  const float y = __builtin_fmaf(e, r, e);
+  const float y = __builtin_amdgcn_fmed3f(__builtin_fmaf(e, r, e), 0.0f, 1.0f);
   const float w = 1.0f + y;
   const float c = y - (w - 1.0f);
   return __builtin_elementwise_maximum(z, 0.0f) + __builtin_fmaf(kLn2, __builtin_amdgcn_logf(w), c);
@@ -393,7 +395,13 @@ int fwd_layers_dispatch(int L, const int* dims, const FwdParams& fp, bool stash,
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, "weight packing kernel launch");
   const bool bf = dtype == MLPMK_DTYPE_BF16;
-  // Tiles of 64 rows where that still gives every CU one, else of 32 rows.
+  // Tiles of 64 rows as soon as tiles of 32 would give a CU a second one.  Up to
+  // 64 rows per CU that leaves CUs without a tile, but each reads the weights
+  // once where two tiles read them twice (64-row / 32-row tiles, us, replayed
+  // graph, 256 CUs): 128-512-512-128 at 9,000 rows 24.1 / 27.3, 16,000 25.6 / 28.8;
+  // 512-512-512-512-512 41.8 / 51.3, 49.8 / 59.3; 6 x 128 20.5 / 23.7, 20.9 / 24.0;
+  // 8 x 32 21.5 / 21.6; only 128-320-320-128 is better off in two: 20.9 / 19.5,
+  // 21.4 / 19.0 (five feature groups of eight waves).
   return fp.M > (int64_t)32 * cus ? layers::launch_any<2>(p, bf, stash, cus, st)
                                   : layers::launch_any<1>(p, bf, stash, cus, st);
 }
