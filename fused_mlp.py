@@ -47,8 +47,9 @@ class FusedMLPSoftplus(nn.Module):
         # The network runs in mlpmk.autograd.kernel_dtype(x): the autocast
         # dtype under autocast, else x's own type (bf16, fp16 or fp32; fp32
         # through bf16 hi/lo split operands) and fp16 for anything else;
-        # networks no fused kernel takes (fp32 wider than 128, any wider
-        # than 256) run layer by layer in that type; autograd carries the
+        # networks no megakernel takes (fp32 wider than 128, any wider
+        # than 256) run through mlpmk.fallback in that type (16-bit ones up
+        # to 512 wide in one launch); autograd carries the
         # gradient back through the casts.  Without autograd (no_grad, inference_mode, or
         # nothing requiring grad) this is one plain forward launch, no stash.
         return fused_mlp(x, *self.weights)

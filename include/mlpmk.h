@@ -221,9 +221,9 @@ int mlpmk_fwd_layers(int num_layers, const int* dims, int dtype, const void* x, 
  *   dw[l]            [dims[l], dims[l+1]] fp32, ACCUMULATED into (+=); the
  *                    caller zeroes them for a fresh gradient, or passes
  *                    dtype | MLPMK_BWD_WRITE_DW to have them written (=)
- * Networks of 4 and 5 layers are supported through mlpmk_bwd_ws only (they
- * hand dz between two launches through the workspace); here they return
- * MLPMK_ERR_INVALID_ARG without touching the device.
+ * Networks of 4 and 5 layers are supported through mlpmk_bwd_ws only (those
+ * with a width above 64 hand dz between two launches through the workspace);
+ * here they return MLPMK_ERR_INVALID_ARG without touching the device.
  */
 int mlpmk_bwd(int num_layers, const int* dims, int dtype, const void* x, const void* const* w,
               const float* const* stash, const void* dout, int64_t dout_row_stride, void* dx,
@@ -240,12 +240,15 @@ int mlpmk_bwd(int num_layers, const int* dims, int dtype, const void* x, const v
  *     adding a whole dW with fp32 atomics (~45-65 us at M = 131072: 256
  *     workgroups x 49152 elements from few CUs each);
  *   - the two-pass backward (fp32 tensors, widths above 128, and 16-bit
- *     batches up to 16,384 rows): a data-gradient kernel over 32-row blocks
- *     of the whole chip writes every dz_l into the workspace, then a
- *     weight-gradient kernel whose workgroups own 64 x 64 blocks of one dW_l
- *     and a chunk of rows adds its tiles to dw with fp32 atomics (summation
- *     order not fixed).
- * Networks of 4 and 5 layers run as two launches (all their dgrad weights
+ *     batches up to 16,384 rows): a data-gradient kernel over tiles of 32 or
+ *     64 rows writes every dz_l into the workspace, then a weight-gradient
+ *     kernel whose workgroups own a block (64 x 64 to 128 x 256) of one dW_l
+ *     and a chunk of rows adds it to dw with fp32 atomics (summation order
+ *     not fixed).  16-bit networks wider than 128 first have their weights
+ *     packed for the data-gradient kernel, from 32,768 rows on, where the
+ *     workspace has room for them.
+ * One-pass networks of 4 and 5 layers run in one launch where no width is
+ * above 64, else as two (all their dgrad weights
  * and exchange tiles do not fit one workgroup's 160 KiB of LDS): layers
  * L-1..S, whose fp16 gradient of h_S goes through the first M * 256 bytes
  * of the workspace (rounded up to 256) to layers S-1..0; S = 3 for the
@@ -254,8 +257,9 @@ int mlpmk_bwd(int num_layers, const int* dims, int dtype, const void* x, const v
  *   workspace        device memory, 16-byte aligned, at least the size that
  *                    mlpmk_bwd_workspace_size reports for the same
  *                    (num_layers, dims, dtype, M, dx != NULL) on the current
- *                    device;
- *                    free again once both launches have run (stream order)
+ *                    device; the packed weights, the last part of it, may be
+ *                    missing (the call then reads the weights in place);
+ *                    free again once the launches have run (stream order)
  */
 int mlpmk_bwd_ws(int num_layers, const int* dims, int dtype, const void* x, const void* const* w,
                  const float* const* stash, const void* dout, int64_t dout_row_stride, void* dx,
@@ -275,7 +279,8 @@ int mlpmk_bwd_ws(int num_layers, const int* dims, int dtype, const void* x, cons
  *     MLPMK_NOALLOC_SCRATCH_BYTES return MLPMK_ERR_UNSUPPORTED_SHAPE before
  *     anything is launched.  What fits: every 3-layer and 2-layer network with
  *     16-bit tensors and widths up to 128 at any M (the partials take at most
- *     48 MiB on MI355X); 4- and 5-layer ones up to the M whose dz hand-over
+ *     48 MiB on MI355X), 4- and 5-layer ones too where no width is above 64;
+ *     the other 4- and 5-layer ones up to the M whose dz hand-over
  *     (M x 256 bytes) still fits (M = 65,536 for the 5-layer 128-wide
  *     network); fp32 tensors and widths above 128 up to the M whose
  *     two-pass dz blocks (M x the hidden widths x the element size) fit
@@ -294,9 +299,11 @@ int mlpmk_bwd_noalloc(int num_layers, const int* dims, int dtype, const void* x,
 /*
  * Bytes of workspace mlpmk_bwd_ws needs on the current device: for the
  * one-pass megakernel one fp32 copy of all dW blocks per workgroup of the
- * backward grid, plus for 4- and 5-layer networks the dz block of the
- * hand-over between their two launches; for the two-pass backward the dz of
- * every hidden layer ([M, width], element size of dtype); the larger where
+ * backward grid, plus for 4- and 5-layer networks with a width above 64 the
+ * dz block of the hand-over between their two launches; for the two-pass
+ * backward the dz of every hidden layer ([M, width], element size of dtype)
+ * and, with 16-bit tensors, a width above 128 and 32,768 rows or more, the
+ * packed weights after them (optional: see workspace above); the larger where
  * a call at this M may take either (0 when M == 0).
  */
 int mlpmk_bwd_workspace_size(int num_layers, const int* dims, int dtype, int64_t M, int with_dx, int64_t* bytes);

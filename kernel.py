@@ -107,7 +107,7 @@ def _pick_config(M, K1, N1, N2, N3, fp32=False, num_cus=None):
 
 # (K1, N1, N2, N3, dtype) -> how _fused_mlp_fwd runs it: 0 one fused launch
 # (also every other dtype, which fwd_into rejects with its own message), a
-# positive count of zero columns to pad x with first, -1 layer by layer.  The
+# positive count of zero columns to pad x with first, -1 mlpmk.fallback.fwd.  The
 # library's answer is cached: asking it costs ~2 us of ctypes per call.
 _ROUTES = {}
 

@@ -1041,7 +1041,8 @@ struct BwdWave {
 
 // The runtime-width kernels of at most 64 features keep two waves per SIMD:
 // left to itself the allocator spread over the accumulation registers and one
-// wave (16-64-64-64-4 in fp16 at 262,144 rows 79 -> 71 us).
+// wave (16-64-64-64-4 in fp16 at 262,144 rows 79 -> 71 us, with a combine
+// kernel of then 7.4; by now 60 + 5).
 template <class N, int NW, bool DX, bool SEG>
 __global__ __launch_bounds__(NW * 64, N::gen && N::ksmax() <= 4 ? 2 : 1) void bwd_kernel(BwdParams p) {
   using Gm = BwdGeom<N, NW, DX, SEG>;
@@ -1090,7 +1091,7 @@ __global__ __launch_bounds__(NW * 64, N::gen && N::ksmax() <= 4 ? 2 : 1) void bw
 // Sums the per-workgroup weight-gradient partials into dw.  A workgroup owns
 // COLS consecutive dW elements; its GROUPS thread groups each
 // sum every GROUPS-th partial (consecutive threads, consecutive
-// elements: a wave's load reads 256 contiguous bytes), the group sums meet in
+// elements: a group's load reads 4 COLS contiguous bytes), the group sums meet in
 // LDS, and one thread per element adds the total to dw with a plain
 // read-modify-write -- each element has exactly one owner, so no atomics.
 // COLS x GROUPS: 64 x 8; few elements (a narrow network's, under 512 blocks of
@@ -1374,7 +1375,7 @@ typedef Gen<BNet3L128> GBNet3;
 // The same compiled at width 64, for networks whose layers all fit it: a
 // quarter of the MFMAs and of the accumulators, so that every depth runs in
 // one launch (16-64-64-64-4 in fp16 at 262,144 rows, 128-wide in two launches
-// -> 64-wide: 166 -> 71 us; 48-wide 3-layer with dx at 100,000: 66 -> 32).
+// -> 64-wide, with the combine kernel: 166 -> 65 us; 48-wide 3-layer with dx at 100,000: 66 -> 32).
 template <int L>
 struct GB64;
 template <>

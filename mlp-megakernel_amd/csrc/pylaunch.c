@@ -95,7 +95,7 @@ static int check_bound(void* fn) {
 #define ERR_OUT() \
   if (PyErr_Occurred()) return NULL
 
-/* bind(fwd, bwd, bwd_ws, wn_fwd, wn_bwd): entry-point addresses. */
+/* bind(fwd, bwd, bwd_ws, wn_fwd, wn_bwd, convert): entry-point addresses. */
 static PyObject* py_bind(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
   (void)self;
   if (check_nargs(nargs, 6, "bind")) return NULL;

@@ -150,7 +150,8 @@ def fwd(x, weights, stash=False):
     128, any tensors wider than 256, more than 5 layers, hidden widths that
     are not multiples of 16.  16-bit networks up to 512 wide and 8 layers deep
     run in one launch (``mlpmk_fwd_layers``, after one that packs the weights;
-    128-512-512-128 in fp16 at 16,384 rows 182 us layer by layer, 25 us).
+    128-512-512-128 in fp16 at 16,384 rows 182 us layer by layer, 26 us), but
+    for the narrowest of many rows (``_gemms_faster``).
     The others run layer by layer: ``z = a @ W_l``
     as an fp32 library GEMM (rocBLAS / hipBLASLt through torch; 16-bit
     values are exact in fp32, so this is the fused kernels' fp32
