@@ -115,7 +115,8 @@ def test_layers_small_activations_keep_their_digits():
     # softplus(z) = e^z (1 - e^z / 2 ...) for z << 0: the fp32 stash within a
     # few ulp of the float64 value of the same fp32 z (z = x w exactly: one
     # input feature), as the elementwise kernel of the layer-by-layer path is.
-    # |z| log2 e rounded to fp32 moves e^z by |z| 2^-24 relative: 1.2e-6 at 20.
+    # (The bound allows e^z from one rounded product, 1.2e-6 at z = -20; the test
+    # over the whole range below holds it to 4 ulp.)
     z = torch.linspace(-20, 24, 352, device="cuda").bfloat16()
     x = torch.zeros((4, 8), device="cuda", dtype=torch.bfloat16)
     x[:, 0] = 1
